@@ -296,31 +296,36 @@ __global__ void __launch_bounds__(WN * 64) __attribute__((amdgpu_waves_per_eu(2)
         }
     };
 
-    // One K tile in pipeline slot `buf` (kt % DEPTH). On entry `op` holds step 0's B operands of `cur`, `dq` the
-    // constants of `cur`, `fa` step 0's activation fragments; on exit the same for K tile kt + 1 (slot `nb`). The
-    // tile DEPTH - 1 ahead goes into slot `lb` (that of K tile kt - 1, whose registers and LDS buffer were last
-    // read before the previous barrier).
-    auto iteration = [&](int kt, int buf, int nb, const BTile<T, G, NSW> &cur, const BTile<T, G, NSW> &nxt, BTile<T, G, NSW> &ld, int lb,
-                         Deq<T> (&dq)[NSW], BOps &op, AFr &fa, auto odd) __attribute__((always_inline)) {
-        constexpr bool kOdd = decltype(odd)::value; // KPB = 2: kt is odd (a barrier follows)
-        const int ktn = min(kt + LOOK, nkt - 1); // the last iterations re-request the last tile; nothing reads it
-        load_b(ktn, ld);
-        load_a(ktn, lb);
+    // One K tile in pipeline slot U = kt % DEPTH. On entry `op` holds step 0's B operands of `cur`, `dq` the
+    // constants of `cur`, `fa` step 0's activation fragments; on exit the same for K tile kt + 1. The tile LOOK ahead
+    // goes into slot (U + LOOK) % DEPTH, whose registers and LDS buffer were last read before the previous barrier.
+    // J >= 0: the J-th iteration behind the loop of whole trips. It requests nothing (two tiles ahead with four slots,
+    // KPB = 2, the first one there still does), and its waits count what the loop's iterations left in flight: the
+    // compiler drops weight loads whose registers nobody reads, and a wait that counted them would let the activation
+    // transfers that it is for slip past.
+    auto iteration = [&](int kt, const BTile<T, G, NSW> &cur, const BTile<T, G, NSW> &nxt, BTile<T, G, NSW> &ld, Deq<T> (&dq)[NSW], BOps &op,
+                         AFr &fa, auto u, auto j) __attribute__((always_inline)) {
+        constexpr int U = decltype(u)::value, J = decltype(j)::value;
+        constexpr bool kOdd = U % 2 == 1; // KPB = 2: a barrier follows
+        constexpr bool kRequest = J < 0 || (KPB == 2 && J == 0);
+        constexpr int ISSUED = KPB == 2 ? 0 : J < 0 ? AHEAD : std::max(0, DEPTH - 3 - J) * (NB + ADMA); // after tile kt + 1's activations
+        if constexpr (kRequest) {
+            const int ktn = min(kt + LOOK, nkt - 1); // the loop's last iterations re-request the last tile; nothing reads it
+            load_b(ktn, ld);
+            load_a(ktn, (U + LOOK) % DEPTH);
+        }
 #pragma unroll
         for (int mu = 0; mu < 4; ++mu) {
             BOps on;
             AFr fn;
             if (mu < 3) {
-                read_a(buf, mu + 1, fn);
+                read_a(U, mu + 1, fn);
                 dequant_step(cur, dq, mu + 1, on);
             } else {
-                if constexpr (KPB == 2) {
-                    // nxt's weights: at an odd kt they were requested one iteration ago, before nxt's and this
-                    // iteration's transfers; at an even kt the barrier before this iteration already waited for them.
-                    wait_vmcnt<kOdd ? 2 * ADMA + NB : ADMA + NB>();
-                } else {
-                    wait_vmcnt<ADMA + AHEAD>(); // nxt's weights (the transfers issued after them may still run)
-                }
+                // nxt's weights; what was issued after them may still run. KPB = 2: at an odd kt they were requested one
+                // iteration ago, before nxt's and this iteration's transfers; at an even kt the barrier before this
+                // iteration already waited for them.
+                wait_vmcnt<KPB == 1 ? ADMA + ISSUED : !kOdd ? ADMA + NB : kRequest ? 2 * ADMA + NB : ADMA>();
                 dequant_step(nxt, dq, 0, on);
             }
             // strip-major: the operand of the last strip, finished at the end of the previous step, is needed last
@@ -344,10 +349,10 @@ __global__ void __launch_bounds__(WN * 64) __attribute__((amdgpu_waves_per_eu(2)
         }
         // The next tile's activations: this wave's transfers done, then everyone's.
         if constexpr (KPB == 1 || kOdd) {
-            wait_vmcnt<AHEAD>();
+            wait_vmcnt<ISSUED>();
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         }
-        read_a(nb, 0, fa);
+        read_a((U + 1) % DEPTH, 0, fa);
     };
 
     BTile<T, G, NSW> b[DEPTH];
@@ -355,6 +360,7 @@ __global__ void __launch_bounds__(WN * 64) __attribute__((amdgpu_waves_per_eu(2)
     for (int t = 0; t < LOOK; ++t) {
         load_b(min(t, nkt - 1), b[t]);
         load_a(min(t, nkt - 1), t);
+        __builtin_amdgcn_sched_barrier(0); // the waits below count these in this order
     }
     Deq<T> dq[NSW];
     BOps op;
@@ -369,29 +375,29 @@ __global__ void __launch_bounds__(WN * 64) __attribute__((amdgpu_waves_per_eu(2)
     asm volatile("s_barrier" ::: "memory");
     read_a(0, 0, fa);
     // DEPTH K tiles per trip, so the register sets and LDS buffers rotate without copies.
-    auto one = [&](int k, auto u) __attribute__((always_inline)) {
+    auto one = [&](int k, auto u, auto j) __attribute__((always_inline)) {
         constexpr int U = decltype(u)::value;
-        using Parity = std::integral_constant<bool, U % 2 == 1>;
-        iteration(k, U, (U + 1) % DEPTH, b[U], b[(U + 1) % DEPTH], b[(U + LOOK) % DEPTH], (U + LOOK) % DEPTH, dq, op, fa, Parity{});
+        iteration(k, b[U], b[(U + 1) % DEPTH], b[(U + LOOK) % DEPTH], dq, op, fa, u, j);
     };
+    using Steady = std::integral_constant<int, -1>;
     int kt = 0;
     for (; kt + DEPTH - 1 < nkt; kt += DEPTH) {
-        one(kt, std::integral_constant<int, 0>{});
-        one(kt + 1, std::integral_constant<int, 1>{});
+        one(kt, std::integral_constant<int, 0>{}, Steady{});
+        one(kt + 1, std::integral_constant<int, 1>{}, Steady{});
         if constexpr (DEPTH == 4) {
-            one(kt + 2, std::integral_constant<int, 2>{});
-            one(kt + 3, std::integral_constant<int, 3>{});
+            one(kt + 2, std::integral_constant<int, 2>{}, Steady{});
+            one(kt + 3, std::integral_constant<int, 3>{}, Steady{});
         }
     }
     if (kt < nkt) {
-        one(kt, std::integral_constant<int, 0>{});
+        one(kt, std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
     }
     if constexpr (DEPTH == 4) {
         if (kt + 1 < nkt) {
-            one(kt + 1, std::integral_constant<int, 1>{});
+            one(kt + 1, std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{});
         }
         if (kt + 2 < nkt) {
-            one(kt + 2, std::integral_constant<int, 2>{});
+            one(kt + 2, std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{});
         }
     }
 
