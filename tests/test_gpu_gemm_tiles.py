@@ -30,3 +30,21 @@ def test_short_k_runs(oracle, hm, device, dtype, kt):
         torch.cuda.synchronize()
         assert_close(oracle, host_f64(y), x64 @ wf, dtype, f"{kt} K tiles M={m}")
         assert torch.equal(y, y2)
+
+
+@pytest.mark.parametrize("group", [32, 64, 128])
+def test_bf16_weights_are_rounded_once(oracle, hm, device, group):
+    # The rows of the identity through the GEMM give back the weights it multiplied with: bf16((q - z) s), rounded once from
+    # the exact product, for every nibble position and value, zero points 0..16 and scales over 2^-100 .. 2^100.
+    rng = np.random.default_rng(310 + group)
+    k, n = 256, 512
+    q = rng.integers(0, 16, (k, n), dtype=np.uint8)
+    z = rng.integers(0, 17, (k // group, n), dtype=np.uint8)
+    s = oracle.to_bits((rng.uniform(1, 2, (k // group, n)) * np.exp2(rng.integers(-100, 101, (k // group, n)))).astype(np.float32), "bf16")
+    w = hm.RepackedMatrix.from_logical(*logical_to_device((q, s, z), "bf16", device), group, dtype=torch.bfloat16)
+    x = torch.eye(k, dtype=torch.bfloat16, device=device)
+    y = torch.empty((k, n), dtype=torch.bfloat16, device=device)
+    hm.packed_linear(y, x, w)
+    torch.cuda.synchronize()
+    exact = (q.astype(np.float64) - np.repeat(z, group, 0)) * np.repeat(oracle.from_bits(s, "bf16").astype(np.float64), group, 0)
+    np.testing.assert_array_equal(host_f64(y), oracle.from_bits(oracle.to_bits(exact.astype(np.float32), "bf16"), "bf16").astype(np.float64))
