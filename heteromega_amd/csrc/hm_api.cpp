@@ -240,19 +240,7 @@ hm_status run_linear(const hm::Planes &p, void *y, int64_t ldy, const void *x, i
 // Workspace for any call of M rows over up to n columns (any column range within them) and kt_count K tiles.
 size_t linear_workspace(const hm::Planes &p, int64_t M, int64_t n, int64_t kt_count, bool fused) {
     if (M > kGemvMaxRows) {
-        // A narrower column range has a smaller grid and may split K further: the largest plan over every width
-        // (at most kGemmPartialMax). More K tiles never split less, so kt_count itself bounds the K ranges.
-        hm::GemmCall c;
-        c.w = p;
-        c.m = M;
-        c.kt_count = kt_count;
-        c.fused = fused;
-        size_t need = 0;
-        for (int64_t w = fused ? 64 : 128; w <= n; w += fused ? 64 : 128) {
-            c.n = w;
-            need = std::max(need, hm::plan_gemm(c).partial_bytes);
-        }
-        return need;
+        return hm::gemm_partial_bound(M, fused ? 2 * n : n, kt_count);
     }
     hm::GemvCall c;
     c.w = p;

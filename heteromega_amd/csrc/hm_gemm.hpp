@@ -1,0 +1,50 @@
+// Prefill GEMM: kernel arguments, tile shapes and launches shared by the planner (hm_gemm.hip) and the kernels
+// (hm_gemm_kernel.hpp).
+#pragma once
+
+#include "hm_internal.hpp"
+
+namespace hm {
+
+struct GemmArgs {
+    const uint4 *quant;
+    const uint32_t *meta;
+    const uint16_t *x;
+    uint16_t *y;
+    float *partial; // [splits][m][ncols] fp32 when the K range is split
+    int64_t ldx, ldy;
+    int kt_pitch;
+    int kt_begin, kt_count, splits;
+    int strip_begin;
+    int m;
+    int ncols; // 16 * strips of the call
+    int tiles_m, tiles_n;
+    int accumulate; // plain output: y = round(y + round(sum)) instead of y = round(sum)
+    int group_m;    // tile order: bands of group_m row tiles, column-major inside a band (1: row-major)
+    int xcds;       // XCDs of the device: the dispatcher places workgroup i on XCD i % xcds
+};
+
+// Tile shapes: 16 rbw rows x 32 wn columns, wk K groups of wn waves, depth LDS buffers, kpb K tiles per barrier. All but
+// the last are eight waves, one workgroup per CU (LDS), and differ in how those waves are spread over columns and K.
+struct GemmTile {
+    int rbw, wn, wk, depth, kpb;
+    constexpr int rows() const { return 16 * rbw; }
+    constexpr int cols() const { return 32 * wn; }
+};
+constexpr GemmTile kGemmTiles[] = {
+    // 64 columns, four K groups
+    {2, 2, 4, 3, 1}, {3, 2, 4, 3, 1}, {4, 2, 4, 2, 1},
+    // 128 columns, two K groups
+    {2, 4, 2, 4, 1}, {3, 4, 2, 4, 1}, {4, 4, 2, 4, 1}, {5, 4, 2, 3, 1}, {6, 4, 2, 3, 1}, {7, 4, 2, 2, 1}, {8, 4, 2, 2, 1},
+    // 256 columns, 2 K tiles ahead in 4 buffers, one barrier per 2 K tiles (against one per K tile, the same bits:
+    // Llama-3-8B M = 2048 gate_up 398.0 -> 392.9 us, down 193.9 -> 192.1)
+    {5, 8, 1, 4, 2}, {6, 8, 1, 4, 2}, {7, 8, 1, 4, 2}, {8, 8, 1, 4, 2},
+    // 128 x 128, four waves: two workgroups per CU
+    {8, 4, 1, 2, 1}};
+constexpr int kGemmTileCount = sizeof(kGemmTiles) / sizeof(kGemmTiles[0]);
+
+// The launches of one activation type (hm_gemm_f16.hip, hm_gemm_bf16.hip).
+hipError_t launch_gemm_f16(const GemmArgs &a, int group, bool fused, int cfg, dim3 grid, hipStream_t s);
+hipError_t launch_gemm_bf16(const GemmArgs &a, int group, bool fused, int cfg, dim3 grid, hipStream_t s);
+
+} // namespace hm

@@ -129,17 +129,18 @@ struct GemmCall {
     float *partial = nullptr; // split-K partials (GemmPlan::partial_bytes)
     bool accumulate = false;  // plain output: y = round(y + round(x W))
 };
-// Tile configuration (2: 128 x 256 tiles, 8 waves; 1: 128 x 128, 4 waves; 0: 64 x 128, 4 waves). The GEMM splits
-// K only for grids of under 128 workgroups and 4-wave grids of under 512, with fp32 partials of at most
-// kGemmPartialMax bytes.
+// Launch shape of a GemmCall: tile shape (index into kGemmTiles, hm_gemm.hpp; -1: none), tile grid, K splits and their
+// fp32 partials, at most kGemmPartialMax bytes.
 constexpr size_t kGemmPartialMax = 32u << 20;
 struct GemmPlan {
-    int cfg = 1;
+    int cfg = -1;
     int64_t tiles_m = 0, tiles_n = 0;
-    int64_t splits = 1, kt_per_split = 0;
+    int64_t splits = 1;
     size_t partial_bytes = 0;
 };
 GemmPlan plan_gemm(const GemmCall &c);
+// A bound on the partials of any call of m rows over up to cols columns (fused: gate and up) and kt K tiles.
+size_t gemm_partial_bound(int64_t m, int64_t cols, int64_t kt);
 hipError_t launch_gemm(const GemmCall &c, hipStream_t stream);
 
 // Adds split-K partials [splits][m][ncols] into y [m, ncols] (or, fused, y [m, ncols / 2] = SiLU(gate) * up

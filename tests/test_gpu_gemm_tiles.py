@@ -1,5 +1,6 @@
 """GPU: the MFMA GEMM (more than 16 rows) at the edges of its pipeline and tiles: K runs shorter than the pipeline is deep and with
-every remainder of its unrolled loop, against the float64 oracle."""
+every remainder of its unrolled loop, and row and column counts on both sides of every tile height, with K groups of unequal length
+and K splits, against the float64 oracle."""
 
 import numpy as np
 import pytest
@@ -48,3 +49,45 @@ def test_bf16_weights_are_rounded_once(oracle, hm, device, group):
     torch.cuda.synchronize()
     exact = (q.astype(np.float64) - np.repeat(z, group, 0)) * np.repeat(oracle.from_bits(s, "bf16").astype(np.float64), group, 0)
     np.testing.assert_array_equal(host_f64(y), oracle.from_bits(oracle.to_bits(exact.astype(np.float32), "bf16"), "bf16").astype(np.float64))
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("k,n,group", [(1152, 384, 32), (1408, 128, 64), (2688, 1024, 128), (1024, 6144, 64)])
+def test_tile_edges(oracle, hm, device, k, n, group, dtype):
+    # Rows on both sides of the tile heights (32 to 128 in steps of 16, one tile and several) in a frame that has to stay
+    # untouched; 9, 11 and 21 K tiles do not divide into the K groups and splits, and 128 and 384 columns leave only the
+    # narrow tiles. The second share of a K-split pair adds into its output through the same tiles.
+    rng = np.random.default_rng(330 + k + n)
+    w_np = oracle.random_weights(rng, k, n, group, dtype)
+    w = hm.RepackedMatrix.from_logical(*logical_to_device(w_np, dtype, device), group, dtype=TORCH[dtype])
+    wf = oracle.weights_f64(*w_np, group, dtype)
+    for m in (17, 32, 33, 48, 49, 64, 65, 80, 81, 96, 97, 112, 113, 128, 129, 177, 225, 257, 385):
+        x64, x = make_x(oracle, rng, m, k, dtype, device)
+        frame = torch.full((m + 2, n + 32), 7.0, dtype=TORCH[dtype], device=device)
+        y = frame[1:m + 1, 16:n + 16]
+        hm.packed_linear(y, x, w)
+        torch.cuda.synchronize()
+        assert_close(oracle, host_f64(y), x64 @ wf, dtype, f"linear {k}x{n} g={group} M={m}")
+        y2 = torch.empty((m, n), dtype=TORCH[dtype], device=device)
+        hm.packed_linear_k_split(y2, torch.cat([x, x], dim=1), w, w)
+        torch.cuda.synchronize()
+        assert torch.equal(y2, y + y), (k, n, m)
+        frame[1:m + 1, 16:n + 16] = 7.0
+        assert bool((frame == 7.0).all()), (k, n, m)
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("hidden,inter,group", [(1152, 1408, 128), (2048, 8192, 64)])
+def test_tile_edges_fused(oracle, hm, device, hidden, inter, group, dtype):
+    # The fused gate_up (SwiGLU after the K groups' exchange, or in the split sum) at the tile heights.
+    rng = np.random.default_rng(350 + hidden)
+    ws = [oracle.random_weights(rng, hidden, inter, group, dtype), oracle.random_weights(rng, hidden, inter, group, dtype),
+          oracle.random_weights(rng, inter, hidden, group, dtype)]
+    layer = hm.FfnLayer.from_logical(*(logical_to_device(t, dtype, device) for t in ws), group, dtype=TORCH[dtype])
+    wg, wu = (oracle.weights_f64(*t, group, dtype) for t in ws[:2])
+    for m in (17, 33, 64, 80, 97, 128, 160, 200, 320):
+        x64, x = make_x(oracle, rng, m, hidden, dtype, device)
+        act = layer.gate_up(x)
+        torch.cuda.synchronize()
+        g = x64 @ wg
+        assert_close(oracle, host_f64(act), g / (1 + np.exp(-g)) * (x64 @ wu), dtype, f"gate_up {hidden}x{inter} M={m}")
