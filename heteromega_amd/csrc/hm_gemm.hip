@@ -12,7 +12,7 @@ namespace {
 // concatenated matrix computed alone gives the bits of the whole call.
 constexpr int64_t kFreeRows = 256;
 constexpr int64_t kLongK = 64; // K tiles
-constexpr int64_t kMaxSplits = 16;
+constexpr int64_t kMaxSplits = 12;
 
 bool may_split(int64_t m, int64_t cols, int64_t kt, int64_t cus) {
     const int64_t tiles = (m + 127) / 128 * (cols / 128);
@@ -21,11 +21,11 @@ bool may_split(int64_t m, int64_t cols, int64_t kt, int64_t cus) {
 
 // Estimated time of a launch in us: what a CU's workgroups take one after the other (each run of `its` K tiles at a cost
 // per tile that grows with the rows, plus what filling the pipeline and writing the tile cost), beside the time the weights
-// take to stream, plus the launch, the exchange between K groups and the split sum. The constants are fitted to some 20000
-// measured launches: gate_up, down, Q/K/V and K/V shapes of Llama-3.2-1B, Llama-3-8B and Qwen2.5-14B, 17 to 2048 rows, fp16
-// and bf16, every tile shape and 1 to 12 splits. Over them the shape it picks takes 0.8% longer than the fastest one on
-// average, and 0.89 of the time of the three shapes and the rules by grid size that it replaced (0.52 to 0.75 for the
-// gate_ups of up to 64 rows, which had taken 128-row tiles; none more than 7% slower).
+// take to stream, plus the launch, the exchange between K groups and the split sum. The constants are fitted to some 50000
+// measured launches on three MI355X: gate_up, down, Q/K/V and K/V shapes of Llama-3.2-1B, Llama-3-8B and Qwen2.5-14B, 17 to
+// 2048 rows, fp16 and bf16, every tile shape and 1 to 12 splits. Over them the shape it picks takes 0.9% longer than the
+// fastest one on average (0.5 to 1.3% by card, 1.16 times at worst), and 0.88 of the time of the three shapes and the rules
+// by grid size that it replaced (0.52 to 0.75 for the gate_ups of up to 64 rows, which had taken 128-row tiles).
 double launch_us(const GemmTile &t, int64_t wgs, int64_t its, int64_t cus, double weight_mb, double partial_mb) {
     const double rounds = static_cast<double>((wgs + cus - 1) / cus);
     const double rb = t.rbw, n = static_cast<double>(its);
@@ -33,14 +33,14 @@ double launch_us(const GemmTile &t, int64_t wgs, int64_t its, int64_t cus, doubl
     if (t.wn * t.wk == 4) { // four waves of eight row blocks, two workgroups per CU (alone on its CU one is faster)
         const double pairs = std::floor(rounds / 2), single = rounds - 2 * pairs;
         fixed = 0.5;
-        busy = pairs * (n * 1.70 + 0.3 * rb) + single * (n * 1.05 + 0.3 * rb);
+        busy = pairs * (n * 1.68 + 0.35 * rb) + single * (n * 1.02 + 0.35 * rb);
     } else {
-        const double per = t.wn == 2 ? 0.39 + 0.23 * rb : t.wn == 4 ? 0.49 + 0.155 * rb : 0.69 + 0.11 * rb;
-        fixed = t.wn == 2 ? 3.3 : t.wn == 4 ? 3.0 : 0.9;
-        busy = rounds * (n * per + 0.3 * rb);
+        const double per = t.wn == 2 ? 0.40 + 0.225 * rb : t.wn == 4 ? 0.49 + (t.kpb == 0 ? 0.149 : 0.157) * rb : 0.75 + 0.103 * rb;
+        fixed = t.wn == 2 ? 3.2 : t.wn == 4 ? 2.9 : 0.6;
+        busy = rounds * (n * per + 0.35 * rb);
     }
-    const double stream = weight_mb / 5.5;
-    return fixed + std::sqrt(busy * busy + stream * stream) + (partial_mb > 0 ? 2.5 + 0.31 * partial_mb : 0.0);
+    const double stream = weight_mb / 5.3;
+    return fixed + std::sqrt(busy * busy + stream * stream) + (partial_mb > 0 ? 3.0 + 0.36 * partial_mb : 0.0);
 }
 
 GemmPlan plan_uncached(int64_t m, int64_t cols, int64_t kt, int64_t cus) {
@@ -55,9 +55,10 @@ GemmPlan plan_uncached(int64_t m, int64_t cols, int64_t kt, int64_t cus) {
         }
         const int64_t tiles_m = (m + t.rows() - 1) / t.rows(), tiles_n = cols / t.cols();
         for (int64_t s = 1; s <= (free ? kMaxSplits : 1); ++s) {
-            // at least two K tiles per run (one run of any length: one K group, no split), partials within their bound
+            // At least two K tiles per run of a K group, four of a lone one (but one run of any length); partials within
+            // their bound.
             const size_t partial = s > 1 ? static_cast<size_t>(s * m * cols) * sizeof(float) : 0;
-            if ((s * t.wk > 1 && kt < 2 * s * t.wk) || partial > kGemmPartialMax) {
+            if ((s * t.wk > 1 && kt < s * (t.wk > 1 ? 2 * t.wk : 4)) || partial > kGemmPartialMax) {
                 break;
             }
             const double us = launch_us(t, tiles_m * tiles_n * s, (kt + s * t.wk - 1) / (s * t.wk), cus, weight_mb, static_cast<double>(partial) * 1e-6);

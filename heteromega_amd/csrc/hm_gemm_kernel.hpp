@@ -136,7 +136,8 @@ __global__ void __launch_bounds__(WN * WK * 64) __attribute__((amdgpu_waves_per_
     constexpr int SPG = 4 / GPT;                  // 32-K steps per group
     constexpr int TRANSFERS = 4 * RBW;            // 1 KiB activation transfers of one K tile
     constexpr int ADMA = (TRANSFERS + WN - 1) / WN; // per wave (past the last: it is repeated, the same bytes to the same place)
-    static_assert(WK == 1 || ((WK == 2 || WK == 4) && KPB == 1), "K groups");
+    static_assert(WK == 1 || WK == 2 || WK == 4, "K groups");
+    static_assert(WK == 1 || KPB < 2, "K groups whose runs differ by a K tile pass the same barriers");
     // K tiles in flight: DEPTH - 1 tiles ahead of the one being multiplied, each with its weights in registers
     // and its activations in one of DEPTH LDS buffers. Per K tile a wave issues NB weight/record loads and ADMA
     // activation transfers, in that order; all of them count in vmcnt, in order.
@@ -144,24 +145,30 @@ __global__ void __launch_bounds__(WN * WK * 64) __attribute__((amdgpu_waves_per_
     // KPB = 2: one barrier per two K tiles. Four LDS buffers, K tiles requested two ahead; the barrier after each odd
     // K tile waits for everything in flight (the next two tiles), and the buffer an iteration fills two tiles ahead was
     // last read before the previous barrier.
-    static_assert(KPB == 1 || (KPB == 2 && DEPTH == 4), "two K tiles per barrier: four buffers");
-    constexpr int LOOK = KPB == 2 ? 2 : DEPTH - 1; // K tiles requested ahead of the one being multiplied
+    // KPB = 0: half tiles. The four LDS buffers hold activations of 64 K each and are refilled every half tile (two
+    // barriers per K tile), so that with the bytes of two whole tiles a transfer has 1.25 K tiles' time instead of one;
+    // weights are requested two K tiles ahead.
+    static_assert(KPB == 1 || DEPTH == 4, "two K tiles per barrier and half tiles: four buffers");
+    constexpr bool kHalf = KPB == 0;
+    constexpr int LOOK = KPB == 1 ? DEPTH - 1 : 2; // K tiles requested ahead of the one being multiplied
     constexpr int NB = 2 * NSW;
+    constexpr int HDMA = (TRANSFERS / 2 + WN - 1) / WN; // transfers per wave per half tile
+    constexpr int BUF = WK * BM * (kHalf ? 128 : 256);  // bytes of an LDS buffer
     constexpr int AHEAD = KPB == 2 ? 0 : (DEPTH - 2) * (NB + ADMA); // loads issued after tile kt + 1's activations at iteration kt
     // Activation tile of one K tile: BM rows of 128 halves (256 B), 16-byte chunks XOR-swizzled by row
     // (chunk c of row r at slot c ^ (r % 16)), so the 16 rows one MFMA operand read touches fall on distinct banks.
     // Two separate arrays (not one [2][...]) so that the compiler can tell the buffers apart and does not
     // make reads of one wait for the transfers into the other.
-    __shared__ __align__(1024) uint8_t as0[WK * BM * 256];
-    __shared__ __align__(1024) uint8_t as1[WK * BM * 256];
-    __shared__ __align__(1024) uint8_t as2[DEPTH > 2 ? WK * BM * 256 : 16];
-    __shared__ __align__(1024) uint8_t as3[DEPTH > 3 ? WK * BM * 256 : 16];
+    __shared__ __align__(1024) uint8_t as0[BUF];
+    __shared__ __align__(1024) uint8_t as1[BUF];
+    __shared__ __align__(1024) uint8_t as2[DEPTH > 2 ? BUF : 16];
+    __shared__ __align__(1024) uint8_t as3[DEPTH > 3 ? BUF : 16];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = uniform(tid >> 6) % WN; // column position
     const int kg = uniform(tid >> 6) / WN;   // K group
-    auto abuf = [&](int buf) __attribute__((always_inline)) { return (buf == 0 ? as0 : buf == 1 ? as1 : buf == 2 ? as2 : as3) + kg * (BM * 256); };
+    auto abuf = [&](int buf) __attribute__((always_inline)) { return (buf == 0 ? as0 : buf == 1 ? as1 : buf == 2 ? as2 : as3) + kg * (BUF / WK); };
     const int col = lane & 15;
     const int h = lane >> 4;
 
@@ -211,12 +218,15 @@ __global__ void __launch_bounds__(WN * WK * 64) __attribute__((amdgpu_waves_per_
                                                   static_cast<uint32_t>(rows_here - 1) * ldx2 + static_cast<uint32_t>(nkt) * 256u);
     // Transfer j of this wave fills LDS bytes [(wave * ADMA + j) KiB, +1 KiB): lane l -> slot p = 64 (wave ADMA + j) + l,
     // row p / 16, swizzled chunk p % 16 (so source chunk (p % 16) ^ (row % 16)). Rows past M read row M - 1.
-    uint32_t xoff[ADMA];
+    // Half tiles: rows of 8 chunks, row p / 8, chunk (p % 8) ^ (row / 2 % 8), so that 16 rows again fall on 16 distinct slots.
+    constexpr int XN = kHalf ? HDMA : ADMA;
+    constexpr int XT = kHalf ? TRANSFERS / 2 : TRANSFERS;
+    uint32_t xoff[XN];
 #pragma unroll
-    for (int j = 0; j < ADMA; ++j) {
-        const int p = min(wave * ADMA + j, TRANSFERS - 1) * 64 + lane;
-        const int r = p >> 4;
-        const int c = (p & 15) ^ (r & 15);
+    for (int j = 0; j < XN; ++j) {
+        const int p = min(wave * XN + j, XT - 1) * 64 + lane;
+        const int r = kHalf ? p >> 3 : p >> 4;
+        const int c = kHalf ? (p & 7) ^ ((r >> 1) & 7) : (p & 15) ^ (r & 15);
         xoff[j] = static_cast<uint32_t>(min(r, rows_here - 1)) * ldx2 + static_cast<uint32_t>(c) * 16u;
     }
     const uint32_t qoff = static_cast<uint32_t>(lane) * 16u;
@@ -246,12 +256,12 @@ __global__ void __launch_bounds__(WN * WK * 64) __attribute__((amdgpu_waves_per_
             bt.w[s] = __builtin_amdgcn_raw_buffer_load_b128(qr, qoff + s * qstrip, static_cast<uint32_t>(kt) * 1024u, 0);
         }
     };
-    // Activation chunks of K tile kt straight into LDS buffer buf (no registers).
+    // Activation chunks of K tile (half tiles: of half tile) kt straight into LDS buffer buf (no registers).
     auto load_a = [&](int kt, int buf) __attribute__((always_inline)) {
-        const uint32_t so = static_cast<uint32_t>(kt) * 256u;
+        const uint32_t so = static_cast<uint32_t>(kt) * (kHalf ? 128u : 256u);
 #pragma unroll
-        for (int j = 0; j < ADMA; ++j) {
-            lds_dma16(xr, abuf(buf) + min(wave * ADMA + j, TRANSFERS - 1) * 1024, xoff[j], so);
+        for (int j = 0; j < XN; ++j) {
+            lds_dma16(xr, abuf(buf) + min(wave * XN + j, XT - 1) * 1024, xoff[j], so);
         }
     };
 
@@ -285,12 +295,12 @@ __global__ void __launch_bounds__(WN * WK * 64) __attribute__((amdgpu_waves_per_
         }
     };
     // Fragment of row block rb, step mu: row rb * 16 + col, chunk 4 mu + h at its swizzled slot.
-    const uint32_t aread = static_cast<uint32_t>(col) * 256u;
+    const uint32_t aread = static_cast<uint32_t>(col) * (kHalf ? 128u : 256u);
     auto read_a = [&](int buf, int mu, AFr &f) __attribute__((always_inline)) {
-        const uint8_t *ab = abuf(buf) + aread + (((4 * mu + h) ^ col) << 4);
+        const uint8_t *ab = abuf(buf) + aread + (((4 * mu + h) ^ (kHalf ? col >> 1 : col)) << 4);
 #pragma unroll
         for (int rb = 0; rb < RBW; ++rb) {
-            f.v[rb] = *reinterpret_cast<const uint4 *>(ab + rb * 4096);
+            f.v[rb] = *reinterpret_cast<const uint4 *>(ab + rb * (kHalf ? 2048 : 4096));
         }
     };
 
@@ -312,6 +322,18 @@ __global__ void __launch_bounds__(WN * WK * 64) __attribute__((amdgpu_waves_per_
             load_b(ktn, ld);
             load_a(ktn, (U + LOOK) % DEPTH);
         }
+        // The next tile's activations: this wave's transfers done, then everyone's (KPB = 2: after each odd tile, for the
+        // next two). Every read of this tile is done too, so the slot that the next iteration fills is free. With tiles
+        // requested two or more ahead this stands before the last step's MFMAs, which then cover the LDS latency of the
+        // next tile's first fragments (against behind them, the same bits: Llama-3-8B layer at M = 2048 586 -> 578 us, at
+        // 512 180 -> 177); with one tile ahead the transfers need the whole iteration (M = 100, 200: 3% slower there).
+        constexpr bool kEarly = DEPTH > 2;
+        auto next_tile = [&]() __attribute__((always_inline)) {
+            if constexpr (KPB == 1 || kOdd) {
+                wait_vmcnt<ISSUED>();
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            }
+        };
 #pragma unroll
         for (int mu = 0; mu < 4; ++mu) {
             BOps on;
@@ -324,6 +346,10 @@ __global__ void __launch_bounds__(WN * WK * 64) __attribute__((amdgpu_waves_per_
                 // iteration ago, before nxt's and this iteration's transfers; at an even kt the barrier before this
                 // iteration already waited for them.
                 wait_vmcnt<KPB == 1 ? ADMA + ISSUED : !kOdd ? ADMA + NB : kRequest ? 2 * ADMA + NB : ADMA>();
+                if constexpr (kEarly) {
+                    next_tile();
+                    read_a((U + 1) % DEPTH, 0, fn);
+                }
                 dequant_step(nxt, dq, 0, on);
             }
             // strip-major: the operand of the last strip, finished at the end of the previous step, is needed last
@@ -341,41 +367,115 @@ __global__ void __launch_bounds__(WN * WK * 64) __attribute__((amdgpu_waves_per_
             }
             __builtin_amdgcn_sched_barrier(0);
             op = on;
-            if (mu < 3) {
+            if (mu < 3 || kEarly) {
                 fa = fn;
             }
         }
-        // The next tile's activations: this wave's transfers done, then everyone's.
-        if constexpr (KPB == 1 || kOdd) {
-            wait_vmcnt<ISSUED>();
-            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if constexpr (!kEarly) {
+            next_tile();
+            read_a((U + 1) % DEPTH, 0, fa);
         }
-        read_a((U + 1) % DEPTH, 0, fa);
+    };
+
+    // Half tiles: the same over the half tiles 2 kt and 2 kt + 1 in LDS buffers 2 U % 4 and the next one. Half tile 2 kt + 3
+    // goes where 2 kt - 1 was, 2 kt + 4 where 2 kt was, each behind the barrier after that one's last read.
+    auto iteration_half = [&](int kt, const BTile<T, G, NSW> &cur, const BTile<T, G, NSW> &nxt, BTile<T, G, NSW> &ld, Deq<T> (&dq)[NSW], BOps &op,
+                              AFr &fa, auto u, auto j) __attribute__((always_inline)) {
+        constexpr int U = decltype(u)::value, J = decltype(j)::value;
+        // Behind the loop: only what a later iteration there reads (J = 0: weights two ahead; J = 0, 1: activations).
+        constexpr bool kWeights = J <= 0, kFirst = J <= 1, kSecond = J <= 0;
+#pragma unroll
+        for (int mu = 0; mu < 4; ++mu) {
+            BOps on;
+            AFr fn;
+            if (mu == 0) {
+                if constexpr (kWeights) {
+                    load_b(min(kt + LOOK, nkt - 1), ld);
+                }
+                if constexpr (kFirst) {
+                    load_a(min(2 * kt + 3, 2 * nkt - 1), (2 * U + 3) % 4);
+                }
+            }
+            if (mu == 2) {
+                if constexpr (kSecond) {
+                    load_a(min(2 * kt + 4, 2 * nkt - 1), (2 * U) % 4);
+                }
+            }
+            if (mu == 1) { // half tile 2 kt + 1 landed (issued after it: 2 kt + 2, then this iteration's first requests)
+                wait_vmcnt<J <= 0 ? 2 * HDMA + NB : J == 1 ? 2 * HDMA : 0>();
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            }
+            if (mu == 3) { // half tile 2 kt + 2 landed (after it: this iteration's requests)
+                wait_vmcnt<J <= 0 ? 2 * HDMA + NB : J == 1 ? HDMA : 0>();
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            }
+            read_a((2 * U + (mu + 1) / 2) % 4, (mu + 1) % 2, fn);
+            if (mu < 3) {
+                dequant_step(cur, dq, mu + 1, on);
+            } else {
+                dequant_step(nxt, dq, 0, on);
+            }
+#pragma unroll
+            for (int s = 0; s < NSW; ++s) {
+#pragma unroll
+                for (int rb = 0; rb < RBW; ++rb) {
+                    acc[rb][s] = T::mfma16(fa.v[rb], op.v[s], acc[rb][s]);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < RBW * NSW; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, SHARE, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            op = on;
+            fa = fn;
+        }
     };
 
     BTile<T, G, NSW> b[DEPTH];
+    // The waits below count these in this order.
+    if constexpr (kHalf) {
+        load_b(0, b[0]);
+        __builtin_amdgcn_sched_barrier(0);
+        load_a(0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        load_b(min(1, nkt - 1), b[1]);
+        __builtin_amdgcn_sched_barrier(0);
+        load_a(1, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        load_a(min(2, 2 * nkt - 1), 2);
+        __builtin_amdgcn_sched_barrier(0);
+    } else {
 #pragma unroll
-    for (int t = 0; t < LOOK; ++t) {
-        load_b(min(t, nkt - 1), b[t]);
-        load_a(min(t, nkt - 1), t);
-        __builtin_amdgcn_sched_barrier(0); // the waits below count these in this order
+        for (int t = 0; t < LOOK; ++t) {
+            load_b(min(t, nkt - 1), b[t]);
+            load_a(min(t, nkt - 1), t);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
     Deq<T> dq[NSW];
     BOps op;
     AFr fa;
-    if constexpr (KPB == 2) {
+    if constexpr (kHalf) {
+        wait_vmcnt<3 * HDMA + NB>();
+    } else if constexpr (KPB == 2) {
         wait_vmcnt<2 * ADMA + NB>(); // tile 0's weights (tile 0's transfers and tile 1's loads may still run)
     } else {
         wait_vmcnt<ADMA + AHEAD>();
     }
     dequant_step(b[0], dq, 0, op);
-    wait_vmcnt<AHEAD>();
+    wait_vmcnt<kHalf ? 2 * HDMA + NB : AHEAD>();
     asm volatile("s_barrier" ::: "memory");
     read_a(0, 0, fa);
     // DEPTH K tiles per trip, so the register sets and LDS buffers rotate without copies.
     auto one = [&](int k, auto u, auto j) __attribute__((always_inline)) {
         constexpr int U = decltype(u)::value;
-        iteration(k, b[U], b[(U + 1) % DEPTH], b[(U + LOOK) % DEPTH], dq, op, fa, u, j);
+        if constexpr (kHalf) {
+            iteration_half(k, b[U], b[(U + 1) % DEPTH], b[(U + LOOK) % DEPTH], dq, op, fa, u, j);
+        } else {
+            iteration(k, b[U], b[(U + 1) % DEPTH], b[(U + LOOK) % DEPTH], dq, op, fa, u, j);
+        }
     };
     using Steady = std::integral_constant<int, -1>;
     int kt = 0;
@@ -408,15 +508,24 @@ __global__ void __launch_bounds__(WN * WK * 64) __attribute__((amdgpu_waves_per_
     // row blocks and finishes the other. A group with a K tile less waits here for the others' last barrier.
     constexpr int HALF = WK > 1 ? (RBW + 1) / 2 : RBW;
     if constexpr (WK > 1) {
-        static_assert(WK / 2 * WN * RBW * NSW * 1024 <= WK * BM * 256, "exchange buffer");
+        static_assert(WK / 2 * WN * RBW * NSW * 1024 <= BUF * (kHalf ? 2 : 1), "exchange buffer");
+        // column positions per buffer: all in as0, or (half tiles) the upper half in as1
+        constexpr int PER = kHalf ? WK / 2 * WN / 2 : WK / 2 * WN;
+        auto slot = [&](int pair) __attribute__((always_inline)) {
+            const int i = pair * WN + wave;
+            return reinterpret_cast<float4_t *>(i < PER ? as0 : as1) + i % PER * (RBW * NSW * 64) + lane;
+        };
         const int longest = base + (split * WK < longer ? 1 : 0); // the split's first run
         if (nkt < longest) {
             asm volatile("s_barrier" ::: "memory");
+            if constexpr (kHalf) {
+                asm volatile("s_barrier" ::: "memory");
+            }
         }
         wait_vmcnt<0>();
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         auto give = [&](int pair, auto lo, auto hi) __attribute__((always_inline)) {
-            float4_t *xch = reinterpret_cast<float4_t *>(as0) + (pair * WN + wave) * (RBW * NSW * 64) + lane;
+            float4_t *xch = slot(pair);
 #pragma unroll
             for (int rb = decltype(lo)::value; rb < decltype(hi)::value; ++rb) {
 #pragma unroll
@@ -426,7 +535,7 @@ __global__ void __launch_bounds__(WN * WK * 64) __attribute__((amdgpu_waves_per_
             }
         };
         auto take = [&](int pair, auto lo, auto hi) __attribute__((always_inline)) {
-            const float4_t *xch = reinterpret_cast<const float4_t *>(as0) + (pair * WN + wave) * (RBW * NSW * 64) + lane;
+            const float4_t *xch = slot(pair);
 #pragma unroll
             for (int rb = decltype(lo)::value; rb < decltype(hi)::value; ++rb) {
 #pragma unroll
