@@ -1202,8 +1202,14 @@ GemvPlan plan_gemv_uncached(const GemvCall &c, int64_t cus, bool allow_few = tru
         // ties go to fewer splits, then to more waves per workgroup. The weights and exponents are fitted to
         // sweeps of every (splits, nu, wps) on the gate_up and down projections of Llama-3-8B, Qwen2.5-14B and
         // Llama-3.2-1B at 2, 4, 8, 12 and 16 rows (one graph of 60 launches per shape, the graphs' replays
-        // interleaved, weights streamed from HBM): the rule's choice is within 5% of the best measured shape on all
-        // 30 of them and 1.1% on average, against 10.8% (at worst 65%) for the rules it replaced.
+        // interleaved, weights streamed from HBM).
+        // Where the whole K does not fit LDS the launch splits in any case, and (groups of 64 and 128) 0.09, 0.03, 0.12 and
+        // 0.13 take those weights' places, fitted to the downs at 9 to 16 rows, fp16 and bf16: more splits, of smaller
+        // staged chunks, two of which fit a CU. The downs run mostly 3 to 6% faster: Llama-3-8B at 16 rows 13.0 -> 12.4 us
+        // (fp16), 13.2 -> 12.5 (bf16), Qwen2.5-14B 14.7 -> 14.2 and 15.0 -> 14.0, Llama-3.2-1B 8.8 -> 8.4 and 8.9 -> 8.6
+        // (groups of 32, half the ring: Llama-3-8B at 6 rows 13.6 -> 15.2, so they keep the first weights).
+        const bool whole = stage_bytes(c.kt_count) <= kLdsMax;
+        const bool deep = !whole && c.w.group > 32;
         const int64_t rows_pad = (c.m + 3) & ~int64_t{3};
         const int gpt = static_cast<int>(128 / c.w.group);
         const int ring = std::max(1, (p.spw == 1 || gpt > 1 ? 4 : 8) / p.spw / (gpt == 4 ? 2 : 1)); // the kernel's KB
@@ -1229,9 +1235,10 @@ GemvPlan plan_gemv_uncached(const GemvCall &c, int64_t cus, bool allow_few = tru
                     const double imb = static_cast<double>((wgs + cus - 1) / cus * cus) / static_cast<double>(wgs);
                     const double r = inflight / static_cast<double>(kRowsInFlight);
                     const double partial = sp > 1 ? 16.0 * static_cast<double>(sp * c.m) / static_cast<double>(c.kt_count * 128) : 0.0;
-                    const double cost = imb * (r < 1.0 ? std::sqrt(1.0 / r) : std::pow(r, 0.05)) *
-                                        (1.0 + 0.05 * static_cast<double>(rows_pad) / (4.0 * nu * p.spw)) * (1.0 + 0.5 * partial) *
-                                        (1.0 + 0.25 * static_cast<double>(rounds - 1));
+                    const double cost = imb * (r < 1.0 ? std::sqrt(1.0 / r) : std::pow(r, deep ? 0.09 : 0.05)) *
+                                        (1.0 + (deep ? 0.03 : 0.05) * static_cast<double>(rows_pad) / (4.0 * nu * p.spw)) *
+                                        (1.0 + (deep ? 0.12 : 0.5) * partial) *
+                                        (1.0 + (deep ? 0.13 : 0.25) * static_cast<double>(rounds - 1));
                     // Candidates come in order of splits, so equal costs keep fewer splits; within the same
                     // splits an equal cost takes the larger workgroup.
                     const bool lower = best < 0.0 || cost < best * (1.0 - 1e-9);
@@ -1255,6 +1262,33 @@ GemvPlan plan_gemv_uncached(const GemvCall &c, int64_t cus, bool allow_few = tru
             p.wps = 1;
             p.nu = 4;
         }
+        // Narrow projections whose whole K fits LDS run in one unsplit launch: the sum of the partials is a second launch
+        // of 2.5-3 us behind a GEMV of 3-5. Each workgroup takes one strip group over the whole K, with 8 waves of at
+        // least 4 K tiles, else 4. fp16 and fused calls take strip pairs; plain bf16 calls, where lone strips stream
+        // better, single strips (two per workgroup of four waves past one strip per CU), also where the rule above has
+        // pairs and does not split. Past one workgroup per CU the staged rows would go round twice (6144 columns in 384
+        // workgroups: 12.4 us against 8.0 in 192 of two strips), so wider calls keep the rule above. Measured at 9 / 16
+        // rows, groups of 128, split -> unsplit in us:
+        //   K x N        fp16                        bf16
+        //   4096 x 4096  8.2 / 8.6 -> 6.9 / 7.2      8.3 / 8.8 -> 6.1 / 6.6
+        //   4096 x 6144  9.2 / 9.4 -> 7.5 / 7.7      9.2 / 9.5 -> 6.9 / 7.4
+        //   4096 x 1024  7.5 / 7.7 -> 6.3 / 6.7      7.6 / 7.8 -> 5.5 / 5.9
+        //   2048 x 3072  7.8 / 8.0 -> 4.9 / 5.2      7.8 / 8.2 -> 4.8 / 5.0
+        //   1024 x 4096  6.7 / 6.9 -> 4.0 / 4.2      6.7 / 7.1 -> 4.0 / 4.1
+        // A pair's wave streams twice the tiles: few pairs of a long K (8192 x 2048, groups of 64 at 5 rows: 8.3 -> 9.3; in
+        // single strips of bf16 8.5 -> 7.6) or in groups of 32 (4096 x 1024 fused: 7.6 -> 8.5) stay split.
+        // (A plan without few rows is made to see whether the rule above splits.)
+        const bool pairs = (c.fused || c.w.dtype == HM_FP16) && strips % 2 == 0;
+        const int64_t groups = pairs ? strips / 2 : strips;
+        const bool fits = pairs ? groups <= cus && c.kt_count <= 40 && (c.w.group > 32 || 4 * groups >= 3 * cus)
+                                : groups <= 2 * cus && c.kt_count <= 64;
+        if (allow_few && whole && fits && (p.splits > 1 || (!pairs && c.kt_count >= 8))) {
+            p.spw = pairs ? 2 : 1;
+            p.groups = groups;
+            set_splits(1);
+            p.nu = groups <= cus ? 1 : 2;
+            p.wps = p.nu == 1 && c.kt_count >= 32 ? 8 : 4;
+        }
     }
     p.waves = p.units > 0 ? p.units : p.nu * p.wps;
     const size_t stage = stage_bytes(p.kt_per_split);
@@ -1271,15 +1305,15 @@ GemvPlan plan_gemv_uncached(const GemvCall &c, int64_t cus, bool allow_few = tru
     return p;
 }
 
-// The plan's inputs: the call's rows, columns, K tiles, fusion, group, pair spill and pair units, and the device's
+// The plan's inputs: the call's rows, columns, K tiles, fusion, group, type, pair spill and pair units, and the device's
 // CU count.
 struct PlanKey {
     int64_t m, n, kt_count, cus;
-    int32_t group, pair_units;
+    int32_t group, pair_units, dtype;
     bool fused, spill;
     bool operator==(const PlanKey &o) const {
         return m == o.m && n == o.n && kt_count == o.kt_count && cus == o.cus && group == o.group && pair_units == o.pair_units &&
-               fused == o.fused && spill == o.spill;
+               dtype == o.dtype && fused == o.fused && spill == o.spill;
     }
 };
 struct PlanKeyHash {
@@ -1287,6 +1321,7 @@ struct PlanKeyHash {
         uint64_t h = 1469598103934665603ull;
         for (const uint64_t v : {static_cast<uint64_t>(k.m), static_cast<uint64_t>(k.n), static_cast<uint64_t>(k.kt_count),
                                  static_cast<uint64_t>(k.cus), static_cast<uint64_t>(k.group), static_cast<uint64_t>(k.pair_units),
+                                 static_cast<uint64_t>(k.dtype),
                                  static_cast<uint64_t>(k.fused) | (static_cast<uint64_t>(k.spill) << 1)}) {
             h = (h ^ v) * 1099511628211ull;
         }
@@ -1300,8 +1335,8 @@ struct PlanKeyHash {
 // host, and each call plans twice), so repeated eager calls of one shape plan once.
 GemvPlan plan_gemv(const GemvCall &c) {
     const int64_t cus = device_topology().cus;
-    const PlanKey key{c.m, c.n, c.kt_count, cus, static_cast<int32_t>(c.w.group), static_cast<int32_t>(c.pair_units), c.fused,
-                      c.pair_spill != nullptr};
+    const PlanKey key{c.m, c.n, c.kt_count, cus, static_cast<int32_t>(c.w.group), static_cast<int32_t>(c.pair_units),
+                      static_cast<int32_t>(c.w.dtype), c.fused, c.pair_spill != nullptr};
     thread_local std::unordered_map<PlanKey, GemvPlan, PlanKeyHash> cache;
     const auto it = cache.find(key);
     if (it != cache.end()) {
@@ -1326,9 +1361,10 @@ size_t gemv_pair_spill_bytes(int64_t channels) {
 
 size_t gemv_partial_bound(const GemvCall &c) {
     // With several rows a split launch has at most kUnitsPerCu (strip group, split) units per CU, whatever range
-    // of the call's columns it covers.
+    // of the call's columns it covers (strip pairs where the strips are even, also if this call itself runs unsplit).
     const GemvPlan p = plan_gemv(c);
-    const size_t narrow = c.m > 1 ? static_cast<size_t>(kUnitsPerCu * device_topology().cus) * p.spw * c.m * 16 * sizeof(float) : 0;
+    const int64_t spw = c.fused || (!p.few && c.n / 16 % 2 == 0) ? 2 : 1;
+    const size_t narrow = c.m > 1 ? static_cast<size_t>(kUnitsPerCu * device_topology().cus) * spw * c.m * 16 * sizeof(float) : 0;
     return std::max(p.partial_bytes, narrow);
 }
 
