@@ -303,7 +303,7 @@ def prefill_gate_up_roofline(hm, torch, dev, layers, m, h, i, replays):
     sec = event_time_graph(torch, g, replays) / len(sets)
     flops = 2.0 * m * h * 2 * i
     achieved = flops / sec / 1e12
-    return {"kernel": "gemm_kernel<F16, 128, true, 8, 2, 8, 4, 2> (fused gate_up + SwiGLU, 128 x 256 tiles, one barrier per two K tiles)", "bound": "mfma",
+    return {"kernel": "gemm_kernel<F16, 128, true, 8, 2, 8, 1, 4, 2> (fused gate_up + SwiGLU, 128 x 256 tiles, one barrier per two K tiles)", "bound": "mfma",
             "achieved": round(achieved, 1), "peak": MFMA_F16_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": round(achieved / MFMA_F16_PEAK_TFLOPS, 4),
             "traffic": measured_traffic(PREFILL_TRAFFIC, "traffic_bytes_per_launch"), "avg_launch_us": round(sec * 1e6, 2),
             "algorithmic_flops_per_launch": int(flops), "rows": m,
