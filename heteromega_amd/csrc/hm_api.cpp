@@ -19,7 +19,7 @@ struct hm_weights {
     void *buffer = nullptr;
     int64_t bytes = 0;
     int64_t quant_bytes = 0, meta_bytes = 0;
-    uint32_t *status = nullptr; // device word after the planes: the repack's out-of-range zero flag
+    uint32_t *status = nullptr; // device word after the planes: what the repack found (kRepackBadZero, kRepackLargeScale)
     bool fused = false;         // gate_up: strips alternate gate / up per 16 channels (N = 2 x channels)
 };
 
@@ -82,7 +82,7 @@ hm_status alloc_planes(hm_weights *w, int64_t K, int64_t N, int64_t group, int d
     return HM_OK;
 }
 
-// Clears the zero-point flag before a repack (load time only, never inside a captured graph).
+// Clears the status word before a repack (load time only, never inside a captured graph).
 hm_status begin_repack(hm_weights *w, hipStream_t s) {
     const hipError_t e = hipMemsetAsync(w->status, 0, sizeof(uint32_t), s);
     return e == hipSuccess ? HM_OK : hip_fail(e, "clearing the repack status");
@@ -91,7 +91,8 @@ hm_status begin_repack(hm_weights *w, hipStream_t s) {
 // Waits for the repack and reports zero points outside 0..16: the kernels read zeros as unsigned bytes and build
 // 1024 + z and 1024 + 16 z in fp16, exact only for small z; the reference's GPU reads tile zeros as int8
 // (w4a16_gemv_packed.cu:86-87) and its CPU as uint8 (w4a16_gemv_avx_packed.cpp:122-124), which agree on 0..127.
-hm_status end_repack(const hm_weights *w, hipStream_t s, const char *what) {
+// Large bf16 scales are kept and noted in the planes: the GEMM dequantizes such a matrix another way.
+hm_status end_repack(hm_weights *w, hipStream_t s, const char *what) {
     uint32_t flag = 0;
     hipError_t e = hipMemcpyAsync(&flag, w->status, sizeof(flag), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) {
@@ -100,9 +101,10 @@ hm_status end_repack(const hm_weights *w, hipStream_t s, const char *what) {
     if (e != hipSuccess) {
         return hip_fail(e, "repack");
     }
-    if (flag != 0) {
+    if (flag & hm::kRepackBadZero) {
         return fail(HM_INVALID_ARGUMENT, "%s: zero points must lie in 0..%u", what, hm::kMaxZero);
     }
+    w->p.large_scales = w->p.dtype == HM_BF16 && (flag & hm::kRepackLargeScale);
     return HM_OK;
 }
 
@@ -319,7 +321,7 @@ hm_status new_ffn(int64_t hidden, int64_t inter, int64_t group, hm_dtype dtype, 
     return HM_OK;
 }
 
-// Runs the repack launches of a new layer (launches(flag) enqueues them with the zero-point flag), waits for them
+// Runs the repack launches of a new layer (launches(status) enqueues them with one status word for both matrices), waits for them
 // and publishes the layer, or frees it on any failure.
 template <class Launches> hm_status fill_ffn(hm_ffn *f, hipStream_t s, const char *what, hm_ffn **out, Launches launches) {
     hm_status st = begin_repack(&f->gate_up, s);
@@ -331,6 +333,7 @@ template <class Launches> hm_status fill_ffn(hm_ffn *f, hipStream_t s, const cha
         destroy_ffn(f);
         return st;
     }
+    f->down.p.large_scales = f->gate_up.p.large_scales;
     for (int64_t m = 1; m <= kGemvMaxRows; ++m) {
         const size_t d = linear_workspace(f->down.p, m, f->hidden, f->inter / 128, false);
         const size_t g = linear_workspace(f->gate_up.p, m, f->inter, f->hidden / 128, true);
@@ -718,6 +721,7 @@ hm_status hm_weights_concat(const hm_weights *const *parts, int32_t count, void 
             delete c;
             return hip_fail(e, "hm_weights_concat copy");
         }
+        c->p.large_scales = c->p.large_scales || w->p.large_scales;
         qo += w->quant_bytes;
         mo += w->meta_bytes;
     }

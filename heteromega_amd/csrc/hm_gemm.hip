@@ -43,14 +43,14 @@ double launch_us(const GemmTile &t, int64_t wgs, int64_t its, int64_t cus, doubl
     return fixed + std::sqrt(busy * busy + stream * stream) + (partial_mb > 0 ? 3.0 + 0.36 * partial_mb : 0.0);
 }
 
-GemmPlan plan_uncached(int64_t m, int64_t cols, int64_t kt, int64_t cus) {
+GemmPlan plan_uncached(int64_t m, int64_t cols, int64_t kt, int64_t cus, bool large_scales) {
     const bool free = may_split(m, cols, kt, cus);
     const double weight_mb = static_cast<double>(kt * 128 * cols) * 0.535e-6; // nibbles and records
     GemmPlan best;
     double best_us = 0;
     for (int i = 0; i < kGemmTileCount; ++i) {
         const GemmTile &t = kGemmTiles[i];
-        if (cols % t.cols() != 0 || (!free && t.wk > 1)) {
+        if (cols % t.cols() != 0 || (!free && t.wk > 1) || (large_scales && i != kLargeScaleTile)) {
             continue;
         }
         const int64_t tiles_m = (m + t.rows() - 1) / t.rows(), tiles_n = cols / t.cols();
@@ -82,6 +82,7 @@ GemmPlan plan_uncached(int64_t m, int64_t cols, int64_t kt, int64_t cus) {
 GemmPlan plan_gemm(const GemmCall &c) {
     struct Entry {
         int64_t m = 0, cols = 0, kt = 0, cus = 0;
+        bool large_scales = false;
         GemmPlan plan;
     };
     constexpr size_t kEntries = 64;
@@ -91,8 +92,9 @@ GemmPlan plan_gemm(const GemmCall &c) {
     const uint64_t h = (static_cast<uint64_t>(c.m) * 0x9E3779B97F4A7C15ull) ^ (static_cast<uint64_t>(cols) * 0xC2B2AE3D27D4EB4Full) ^
                        (static_cast<uint64_t>(c.kt_count) * 0x165667B19E3779F9ull);
     Entry &e = cache[(h >> 32) % kEntries];
-    if (e.m != c.m || e.cols != cols || e.kt != c.kt_count || e.cus != cus) {
-        e.plan = plan_uncached(c.m, cols, c.kt_count, cus);
+    if (e.m != c.m || e.cols != cols || e.kt != c.kt_count || e.cus != cus || e.large_scales != c.w.large_scales) {
+        e.plan = plan_uncached(c.m, cols, c.kt_count, cus, c.w.large_scales);
+        e.large_scales = c.w.large_scales;
         e.m = c.m;
         e.cols = cols;
         e.kt = c.kt_count;
@@ -137,8 +139,9 @@ hipError_t launch_gemm(const GemmCall &c, hipStream_t stream) {
     a.xcds = device_topology().xcds;
     const dim3 grid(static_cast<unsigned>(p.tiles_m * p.tiles_n), static_cast<unsigned>(p.splits));
     const int group = static_cast<int>(c.w.group);
-    const hipError_t e = c.w.dtype == HM_FP16 ? launch_gemm_f16(a, group, c.fused, p.cfg, grid, stream)
-                                              : launch_gemm_bf16(a, group, c.fused, p.cfg, grid, stream);
+    const hipError_t e = c.w.dtype == HM_FP16  ? launch_gemm_f16(a, group, c.fused, p.cfg, grid, stream)
+                         : c.w.large_scales ? launch_gemm_bf16_large_scales(a, group, c.fused, grid, stream)
+                                            : launch_gemm_bf16(a, group, c.fused, p.cfg, grid, stream);
     if (e != hipSuccess || p.splits == 1) {
         return e;
     }

@@ -45,9 +45,13 @@ constexpr GemmTile kGemmTiles[] = {
     // 128 x 128, four waves: two workgroups per CU (half tiles for the same reason: 2-7% faster at 640 rows)
     {8, 4, 1, 4, 0}};
 constexpr int kGemmTileCount = sizeof(kGemmTiles) / sizeof(kGemmTiles[0]);
+// The tile of bf16 matrices with scales from 2^117 on (Planes::large_scales): the only one that their dequantization is built for.
+constexpr int kLargeScaleTile = kGemmTileCount - 1;
+static_assert(kGemmTiles[kLargeScaleTile].cols() == 128 && kGemmTiles[kLargeScaleTile].wk == 1, "fits every call");
 
 // The launches of one activation type (hm_gemm_f16.hip, hm_gemm_bf16.hip).
 hipError_t launch_gemm_f16(const GemmArgs &a, int group, bool fused, int cfg, dim3 grid, hipStream_t s);
 hipError_t launch_gemm_bf16(const GemmArgs &a, int group, bool fused, int cfg, dim3 grid, hipStream_t s);
+hipError_t launch_gemm_bf16_large_scales(const GemmArgs &a, int group, bool fused, dim3 grid, hipStream_t s); // in kLargeScaleTile
 
 } // namespace hm

@@ -2,5 +2,5 @@
 #include "hm_gemm_kernel.hpp"
 
 hipError_t hm::launch_gemm_f16(const GemmArgs &a, int group, bool fused, int cfg, dim3 grid, hipStream_t s) {
-    return launch_t<F16>(a, group, fused, cfg, grid, s);
+    return launch_t<F16>(a, group, fused, cfg, grid, s, AllTiles{});
 }

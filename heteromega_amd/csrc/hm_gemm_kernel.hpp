@@ -60,9 +60,14 @@ template <> struct Deq<F16> {
     uint32_t d2, s2, d2w, s2w;
 };
 // bf16: s, -(1024 + z) s and, for the wide positions, s / 16 and -(1024 + 16 z) s / 16 in fp32 (all exact for scales
-// of 2^-114 to 2^117).
+// below 2^117).
 template <> struct Deq<BF16> {
     float s, d, sw, dw;
+};
+// bf16 matrices with scales from 2^117 on, where 1024 s leaves fp32: s and z.
+struct BF16Large : BF16 {};
+template <> struct Deq<BF16Large> {
+    float s, z;
 };
 
 __device__ __forceinline__ Deq<F16> make_deq(uint32_t rec, F16) {
@@ -80,6 +85,10 @@ __device__ __forceinline__ Deq<BF16> make_deq(uint32_t rec, BF16) {
     const float z = static_cast<float>((rec >> 16) & 0xFFu);
     const float sw = 0.0625f * s;
     return Deq<BF16>{s, (-1024.0f - z) * s, sw, __builtin_fmaf(z, -s, -1024.0f * sw)};
+}
+
+__device__ __forceinline__ Deq<BF16Large> make_deq(uint32_t rec, BF16Large) {
+    return Deq<BF16Large>{bf16_bits_to_float(rec & 0xFFFFu), static_cast<float>((rec >> 16) & 0xFFu)};
 }
 
 // B operand of one 32-K step from one strip dword: (q - z) * s in the activation type.
@@ -121,6 +130,19 @@ __device__ __forceinline__ uint4 dequant_operand(uint32_t w, const Deq<BF16> &q,
     // dword i holds K elements 2i, 2i + 1 (nibbles i and 4 + i)
     return uint4{pair((w & m.lo) | m.magic, q.s, q.d), pair((w & m.hi) | m.magic, q.sw, q.dw), pair((u & m.lo) | m.magic, q.s, q.d),
                  pair((u & m.hi) | m.magic, q.sw, q.dw)};
+}
+
+// bf16 with large scales: (q - z) s by a subtraction and a product in fp32, both exact while the weight is finite, for any
+// scale. Such matrices hardly exist, so this one is built for a single tile and not tuned.
+__device__ __forceinline__ uint4 dequant_operand(uint32_t w, const Deq<BF16Large> &q, const MagicRegs &) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    // dword i holds K elements 2i, 2i + 1 (nibbles i and 4 + i)
+    auto pair = [&](int i) __attribute__((always_inline)) {
+        const f2 r = {(static_cast<float>((w >> (4 * i)) & 0xFu) - q.z) * q.s, (static_cast<float>((w >> (4 * i + 16)) & 0xFu) - q.z) * q.s};
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector(r, b2));
+    };
+    return uint4{pair(0), pair(1), pair(2), pair(3)};
 }
 
 template <class T, int G, int NSW> struct BTile {
@@ -648,17 +670,19 @@ hipError_t launch_g(const GemmArgs &a, bool fused, int cfg, dim3 grid, hipStream
     return e;
 }
 
-template <class T> hipError_t launch_t(const GemmArgs &a, int group, bool fused, int cfg, dim3 grid, hipStream_t s) {
-    constexpr auto all = std::make_integer_sequence<int, kGemmTileCount>{};
+// The tiles I... are built; cfg is one of them.
+template <class T, int... I>
+hipError_t launch_t(const GemmArgs &a, int group, bool fused, int cfg, dim3 grid, hipStream_t s, std::integer_sequence<int, I...> tiles) {
     switch (group) {
     case 32:
-        return launch_g<T, 32>(a, fused, cfg, grid, s, all);
+        return launch_g<T, 32>(a, fused, cfg, grid, s, tiles);
     case 64:
-        return launch_g<T, 64>(a, fused, cfg, grid, s, all);
+        return launch_g<T, 64>(a, fused, cfg, grid, s, tiles);
     default:
-        return launch_g<T, 128>(a, fused, cfg, grid, s, all);
+        return launch_g<T, 128>(a, fused, cfg, grid, s, tiles);
     }
 }
+using AllTiles = std::make_integer_sequence<int, kGemmTileCount>;
 
 } // namespace
 

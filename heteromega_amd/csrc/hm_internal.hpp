@@ -28,6 +28,7 @@ struct Planes {
     const uint32_t *meta = nullptr; // (N/16) * (K/group) * 16 records
     int64_t K = 0, N = 0, group = 128;
     int dtype = 0; // hm_dtype
+    bool large_scales = false; // bf16: a scale of kLargeScale or more (finite)
     int64_t kt_pitch() const { return K / 128; }
 };
 
@@ -43,6 +44,10 @@ struct TileSource {
 };
 // Largest zero point the repack accepts (GPTQ checkpoints store z - 1, so z reaches 16 after adding the one back).
 constexpr uint32_t kMaxZero = 16;
+// bf16 scales from 2^117 on (their bits, sign cleared): the GEMM's usual dequantization forms 1040 times the scale in fp32.
+constexpr uint32_t kLargeScaleBits = (117 + 127) << 7;
+// Bits of the repack status word.
+constexpr uint32_t kRepackBadZero = 1, kRepackLargeScale = 2;
 struct LogicalSource {
     const uint8_t *q = nullptr;      // [K, ld] row-major
     const uint16_t *scales = nullptr; // [K/group, ld]
@@ -51,12 +56,13 @@ struct LogicalSource {
 };
 
 // Repack launches. `fused` interleaves two sources per 16 columns (strip 2j from src[0], 2j + 1 from src[1]);
-// then N counts the columns of the result (2x the columns taken from each source). A zero point above kMaxZero
-// sets bit 0 of *bad_zero (device memory, may be null).
+// then N counts the columns of the result (2x the columns taken from each source). *status (device memory) gets
+// kRepackBadZero for a zero point above kMaxZero and kRepackLargeScale for a stored scale whose bits are those of a
+// finite bf16 from kLargeScaleBits on (of no meaning in an fp16 plane).
 hipError_t launch_repack_tiles(const TileSource *src, int nsrc, bool fused, uint8_t *quant, uint32_t *meta, int64_t K,
-                               int64_t N, int dtype, uint32_t *bad_zero, hipStream_t stream);
+                               int64_t N, int dtype, uint32_t *status, hipStream_t stream);
 hipError_t launch_repack_logical(const LogicalSource *src, int nsrc, bool fused, uint8_t *quant, uint32_t *meta,
-                                 int64_t K, int64_t N, int64_t group, uint32_t *bad_zero, hipStream_t stream);
+                                 int64_t K, int64_t N, int64_t group, uint32_t *status, hipStream_t stream);
 hipError_t launch_unpack(const Planes &p, uint8_t *q, uint16_t *scales, uint8_t *zeros, hipStream_t stream);
 // Dequantized weights round((q - z) s) in the activation type: [N, K] (transposed, the orientation of the
 // reference's dequantize_packed) or [K, N], leading dimension ld.

@@ -42,9 +42,11 @@ __device__ __forceinline__ int64_t packed_column(const TileSource &src, int64_t 
     return ((c >> 6) << 7) + (src.col_mode == 2 ? 64 : 0) + (c & 63);
 }
 
-__device__ __forceinline__ void check_zero(uint32_t z, uint32_t *bad_zero) {
-    if (z > kMaxZero && bad_zero != nullptr) {
-        atomicOr(bad_zero, 1u);
+__device__ __forceinline__ void check_record(uint32_t sbits, uint32_t z, uint32_t *status) {
+    const uint32_t magnitude = sbits & 0x7FFFu;
+    const uint32_t found = (z > kMaxZero ? kRepackBadZero : 0u) | (magnitude >= kLargeScaleBits && magnitude < 0x7F80u ? kRepackLargeScale : 0u);
+    if (found != 0) {
+        atomicOr(status, found);
     }
 }
 
@@ -86,7 +88,7 @@ __global__ void __launch_bounds__(256)
 
 __global__ void __launch_bounds__(256)
     repack_tiles_meta(TileSource s0, TileSource s1, bool fused, uint32_t *__restrict__ meta, int64_t kt, int64_t total, int dtype,
-                      uint32_t *bad_zero) {
+                      uint32_t *status) {
     const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     if (idx >= total) {
         return;
@@ -103,8 +105,9 @@ __global__ void __launch_bounds__(256)
     const int cn = static_cast<int>(n_src & 63);
     const uint32_t sbits = static_cast<uint32_t>(tile[4096 + 2 * cn]) | (static_cast<uint32_t>(tile[4096 + 2 * cn + 1]) << 8);
     const uint32_t z = tile[4224 + (cn >> 3) * 16 + (cn & 7)];
-    check_zero(z, bad_zero);
-    meta[idx] = bf16_bits_to_dtype(sbits, dtype) | (z << 16);
+    const uint32_t stored = bf16_bits_to_dtype(sbits, dtype);
+    check_record(stored, z, status);
+    meta[idx] = stored | (z << 16);
 }
 
 __global__ void __launch_bounds__(256)
@@ -134,7 +137,7 @@ __global__ void __launch_bounds__(256)
 
 __global__ void __launch_bounds__(256)
     repack_logical_meta(LogicalSource s0, LogicalSource s1, bool fused, uint32_t *__restrict__ meta, int64_t kt, int gpt, int64_t total,
-                        uint32_t *bad_zero) {
+                        uint32_t *status) {
     const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     if (idx >= total) {
         return;
@@ -150,7 +153,7 @@ __global__ void __launch_bounds__(256)
     const LogicalSource &src = which ? s1 : s0;
     const uint32_t sbits = src.scales[g * src.ld + n_src];
     const uint32_t z = src.zeros[g * src.ld + n_src];
-    check_zero(z, bad_zero);
+    check_record(sbits, z, status);
     meta[idx] = sbits | (z << 16);
 }
 
@@ -239,7 +242,7 @@ dim3 blocks_for(int64_t total) { return dim3(static_cast<unsigned>((total + 255)
 } // namespace
 
 hipError_t launch_repack_tiles(const TileSource *src, int nsrc, bool fused, uint8_t *quant, uint32_t *meta, int64_t K,
-                               int64_t N, int dtype, uint32_t *bad_zero, hipStream_t stream) {
+                               int64_t N, int dtype, uint32_t *status, hipStream_t stream) {
     const TileSource s0 = src[0];
     const TileSource s1 = nsrc > 1 ? src[1] : src[0];
     const int64_t kt = K / 128;
@@ -250,13 +253,13 @@ hipError_t launch_repack_tiles(const TileSource *src, int nsrc, bool fused, uint
     }
     const int64_t records = (N / 16) * kt * 16;
     if (records > 0) {
-        hipLaunchKernelGGL(repack_tiles_meta, blocks_for(records), dim3(256), 0, stream, s0, s1, fused, meta, kt, records, dtype, bad_zero);
+        hipLaunchKernelGGL(repack_tiles_meta, blocks_for(records), dim3(256), 0, stream, s0, s1, fused, meta, kt, records, dtype, status);
     }
     return hipGetLastError();
 }
 
 hipError_t launch_repack_logical(const LogicalSource *src, int nsrc, bool fused, uint8_t *quant, uint32_t *meta,
-                                 int64_t K, int64_t N, int64_t group, uint32_t *bad_zero, hipStream_t stream) {
+                                 int64_t K, int64_t N, int64_t group, uint32_t *status, hipStream_t stream) {
     const LogicalSource s0 = src[0];
     const LogicalSource s1 = nsrc > 1 ? src[1] : src[0];
     const int64_t kt = K / 128;
@@ -269,7 +272,7 @@ hipError_t launch_repack_logical(const LogicalSource *src, int nsrc, bool fused,
     const int64_t records = (N / 16) * groups * 16;
     if (records > 0) {
         hipLaunchKernelGGL(repack_logical_meta, blocks_for(records), dim3(256), 0, stream, s0, s1, fused, meta, kt,
-                           static_cast<int>(128 / group), records, bad_zero);
+                           static_cast<int>(128 / group), records, status);
     }
     return hipGetLastError();
 }

@@ -51,6 +51,71 @@ def test_bf16_weights_are_rounded_once(oracle, hm, device, group):
     np.testing.assert_array_equal(host_f64(y), oracle.from_bits(oracle.to_bits(exact.astype(np.float32), "bf16"), "bf16").astype(np.float64))
 
 
+def _any_scales(rng, oracle, shape, lo, hi):
+    bits = oracle.to_bits((rng.uniform(1, 1.99, shape) * np.exp2(rng.integers(lo, hi, shape))).astype(np.float32), "bf16")
+    return bits, oracle.from_bits(bits, "bf16").astype(np.float64)
+
+
+@pytest.mark.parametrize("group", [32, 64, 128])
+def test_bf16_scales_of_any_size(oracle, hm, device, group):
+    # The weights that the GEMM multiplies with, read back by the rows of the identity, over every bf16 scale: subnormal ones
+    # (from 2^-133) to the largest, where (1024 + z) s leaves fp32 long before the weight leaves bf16. A weight beyond bf16 is
+    # infinite. Also in a matrix joined from one without large scales and one with, and with K splits.
+    rng = np.random.default_rng(320 + group)
+    k, n = 256, 512
+    x = torch.eye(k, dtype=torch.bfloat16, device=device)
+    parts, exact = [], []
+    for lo, hi in ((-133, 117), (-133, 128), (116, 128)):
+        q = rng.integers(0, 16, (k, n), dtype=np.uint8)
+        z = rng.integers(0, 17, (k // group, n), dtype=np.uint8)
+        bits, s = _any_scales(rng, oracle, (k // group, n), lo, hi)
+        w = hm.RepackedMatrix.from_logical(*logical_to_device((q, bits, z), "bf16", device), group, dtype=torch.bfloat16)
+        with np.errstate(over="ignore"):
+            e = ((q.astype(np.float64) - np.repeat(z, group, 0)) * np.repeat(s, group, 0)).astype(np.float32)
+            e = torch.from_numpy(e).to(torch.bfloat16)
+        # one row's product with an infinite weight of another row is 0 * inf: only columns of finite weights come back
+        fine = torch.isfinite(e).all(dim=0)
+        assert bool(fine.any())
+        y = torch.empty((k, n), dtype=torch.bfloat16, device=device)
+        hm.packed_linear(y, x, w)
+        torch.cuda.synchronize()
+        assert torch.equal(y.cpu()[:, fine], e[:, fine]), (lo, hi)
+        parts.append(w)
+        exact.append((e, fine))
+    joined = hm.RepackedMatrix.concat(parts[:2])
+    y = torch.empty((k, 2 * n), dtype=torch.bfloat16, device=device)
+    hm.packed_linear(y, x, joined)
+    torch.cuda.synchronize()
+    for i, (e, fine) in enumerate(exact[:2]):
+        assert torch.equal(y.cpu()[:, i * n:(i + 1) * n][:, fine], e[:, fine])
+
+
+@pytest.mark.parametrize("source", ["logical", "tiles"])
+def test_bf16_large_scales_in_a_layer(oracle, hm, device, source):
+    # Up weights of about 2^120 and down weights of about 2^-100 (one matrix with large scales makes the layer take their
+    # dequantization), a K range that splits, group 128, through both halves of the layer.
+    rng = np.random.default_rng(325)
+    hidden, inter, g, m = 2048, 256, 128, 40
+    mats = [list(oracle.random_weights(rng, *s, g, "bf16")) for s in ((hidden, inter), (hidden, inter), (inter, hidden))]
+    for i, e in ((1, 119), (2, -100)):
+        mats[i][1] = _any_scales(rng, oracle, mats[i][1].shape, e, e + 1)[0]
+    x64, x = make_x(oracle, rng, m, hidden, "bf16", device, scale=2.0 ** -4)
+    if source == "logical":
+        layer = hm.FfnLayer.from_logical(*(logical_to_device(t, "bf16", device) for t in mats), g, dtype=torch.bfloat16)
+    else:
+        packed = [torch.from_numpy(hm.pack_w4a16(q, s, z.astype(np.int8))).to(device) for q, s, z in mats]
+        layer = hm.FfnLayer.from_tiles(*packed, hidden, inter, dtype=torch.bfloat16)
+    act = layer.gate_up(x)
+    y = layer.down(act)
+    torch.cuda.synchronize()
+    wg, wu, wd = (oracle.weights_f64(*t, g, "bf16") for t in mats)
+    gate = x64 @ wg
+    ref = gate / (1 + np.exp(-gate)) * (x64 @ wu)
+    assert np.abs(ref).max() > 2.0 ** 115
+    assert_close(oracle, host_f64(act) * 2.0 ** -118, ref * 2.0 ** -118, "bf16", "gate_up with large scales")
+    assert_close(oracle, host_f64(y), host_f64(act) @ wd, "bf16", "down of the same layer")
+
+
 @pytest.mark.parametrize("dtype", ["fp16", "bf16"])
 @pytest.mark.parametrize("k,n,group", [(1152, 384, 32), (1408, 128, 64), (2688, 1024, 128), (1024, 6144, 64)])
 def test_tile_edges(oracle, hm, device, k, n, group, dtype):
