@@ -6,6 +6,7 @@ packed_linear, gemv_w4a16, gemm_w4a16, silu_mul, residual_add2, GpuFfnModel) and
 TORCH_CHECK / ValueError) and HMError for device failures. torch is used for device memory and streams only.
 """
 
+import contextlib
 import ctypes
 import math
 from numbers import Integral
@@ -44,6 +45,35 @@ def _stream(stream, device=None):
     if isinstance(stream, torch.cuda.Stream):
         return stream.cuda_stream
     return int(stream)
+
+
+def _on(stream, device):
+    """`stream` as torch's current stream, for what a call allocates or computes with torch by itself. A block of the current
+    stream's pool may still be in use there, and a freed one goes back to it at once, while `stream` works on it; a block of
+    `stream`'s own pool is reused in its order."""
+    if stream is None or device.type != "cuda":
+        return contextlib.nullcontext()
+    handle = _stream(stream)
+    if handle == _stream(None, device):
+        return contextlib.nullcontext()
+    if not isinstance(stream, torch.cuda.Stream):
+        # 0 and 1 (hipStreamLegacy) are the default stream
+        stream = torch.cuda.default_stream(device) if handle in (0, 1) else torch.cuda.ExternalStream(handle, device=device)
+    return torch.cuda.stream(stream)
+
+
+def _result(shape, dtype, device, stream):
+    """A new tensor that `stream` writes and the caller, on the current stream, reads and drops."""
+    with _on(stream, device):
+        t = torch.empty(shape, dtype=dtype, device=device)
+    return _handed_over(t, stream)
+
+
+def _handed_over(t, stream):
+    """t, made on `stream`, as a result: its memory is free again once the current stream's work with it is done too."""
+    if stream is not None and t.is_cuda:
+        t.record_stream(torch.cuda.current_stream(t.device))
+    return t
 
 
 def _ptr(t):
@@ -215,7 +245,7 @@ class RepackedMatrix:
         """round((q - z) * s) in the activation type: [N, K] (QuantizedLinearImpl::dequantize_packed's orientation,
         unified_llm_w4a16.cpp:710-790) or [K, N]."""
         shape = (self.n, self.k) if transposed else (self.k, self.n)
-        out = torch.empty(shape, dtype=self.dtype, device=self.device)
+        out = _result(shape, self.dtype, self.device, stream)
         _call(_lib.load().hm_weights_dequantize(self._h, _ptr(out), out.stride(0), 1 if transposed else 0, _stream(stream, self.device)))
         return out
 
@@ -232,9 +262,9 @@ class RepackedMatrix:
         return cls(h, parts[0].device)
 
     def to_logical(self, stream=None):
-        q = torch.empty((self.k, self.n), dtype=torch.uint8, device=self.device)
-        s = torch.empty((self.k // self.group, self.n), dtype=self.dtype, device=self.device)
-        z = torch.empty((self.k // self.group, self.n), dtype=torch.uint8, device=self.device)
+        q = _result((self.k, self.n), torch.uint8, self.device, stream)
+        s = _result((self.k // self.group, self.n), self.dtype, self.device, stream)
+        z = _result((self.k // self.group, self.n), torch.uint8, self.device, stream)
         _call(_lib.load().hm_weights_to_logical(self._h, _ptr(q), _ptr(s), _ptr(z), _stream(stream, self.device)))
         return q, s, z
 
@@ -259,10 +289,12 @@ class RepackedMatrix:
             pass
 
 
-def _workspace(nbytes, device):
+def _workspace(nbytes, device, stream):
+    """Scratch of calls on `stream`."""
     if nbytes == 0:
         return None
-    return torch.empty(nbytes + 256, dtype=torch.uint8, device=device)
+    with _on(stream, device):
+        return torch.empty(nbytes + 256, dtype=torch.uint8, device=device)
 
 
 def _aligned(ws):
@@ -287,7 +319,7 @@ def packed_linear(out, inp, w, k=None, n=None, col_begin=0, stream=None, workspa
     if inp.dtype != w.dtype or out.dtype != w.dtype:
         raise ValueError(f"packed_linear: input and output must be {w.dtype}")
     if workspace is None:
-        workspace = _workspace(w.workspace_bytes(m, k, n), inp.device)
+        workspace = _workspace(w.workspace_bytes(m, k, n), inp.device, stream)
     wp, wb = _aligned(workspace)
     _call(_lib.load().hm_linear(w._h, _ptr(out), out.stride(0), _ptr(inp), inp.stride(0), m, k, n, col_begin, wp, wb,
                                 _stream(stream, inp.device)))
@@ -310,7 +342,7 @@ def packed_linear_k_split(out, inp, w0, w1, k0=None, k1=None, n=None, stream=Non
         raise ValueError(f"packed_linear_k_split: input, output and both shares must be {w0.dtype}")
     lib = _lib.load()
     if workspace is None:
-        workspace = _workspace(lib.hm_linear_k_split_workspace_bytes(w0._h, w1._h, m, k0, k1, n), inp.device)
+        workspace = _workspace(lib.hm_linear_k_split_workspace_bytes(w0._h, w1._h, m, k0, k1, n), inp.device, stream)
     wp, wb = _aligned(workspace)
     _call(lib.hm_linear_k_split(w0._h, w1._h, _ptr(out), out.stride(0), _ptr(inp), inp.stride(0), m, k0, k1, n, wp, wb,
                                 _stream(stream, inp.device)))
@@ -332,7 +364,7 @@ def packed_linear_swiglu(act, inp, w, k=None, channels=None, stream=None, worksp
         raise ValueError(f"packed_linear_swiglu: output must be [M, >= {e - b}]")
     lib = _lib.load()
     if workspace is None:
-        workspace = _workspace(lib.hm_linear_swiglu_workspace_bytes(w._h, m, k, e - b), inp.device)
+        workspace = _workspace(lib.hm_linear_swiglu_workspace_bytes(w._h, m, k, e - b), inp.device, stream)
     wp, wb = _aligned(workspace)
     _call(lib.hm_linear_swiglu(w._h, _ptr(act), act.stride(0), _ptr(inp), inp.stride(0), m, k, b, e, wp, wb, _stream(stream, inp.device)))
     return act
@@ -415,10 +447,11 @@ def find_nonfinite(t, sampled=False, stream=None):
         raise ValueError("find_nonfinite: a [rows, columns] tensor with a contiguous last dimension")
     L = _lib.load()
     if t.is_cuda:
-        first = torch.empty((1,), dtype=torch.int64, device=t.device)
-        _call(L.hm_find_nonfinite_device(_ptr(t), t.size(0), t.size(1), t.stride(0), _hm_dtype(t.dtype), int(bool(sampled)), _ptr(first),
-                                         _stream(stream, t.device)))
-        return int(first.item())
+        with _on(stream, t.device):
+            first = torch.empty((1,), dtype=torch.int64, device=t.device)
+            _call(L.hm_find_nonfinite_device(_ptr(t), t.size(0), t.size(1), t.stride(0), _hm_dtype(t.dtype), int(bool(sampled)), _ptr(first),
+                                             _stream(stream, t.device)))
+            return int(first.item())
     return int(L.hm_find_nonfinite(_ptr(t), t.size(0), t.size(1), t.stride(0), _hm_dtype(t.dtype), int(bool(sampled))))
 
 
@@ -492,8 +525,8 @@ class FfnLayer:
         need = self.workspace_bytes(max_m)
         ws = self._ws.get(key)
         if ws is None or ws.numel() < need + 256:
-            ws = torch.empty(need + 256, dtype=torch.uint8, device=self.device)
-            self._ws[key] = ws
+            with _on(stream, self.device):
+                ws = self._ws[key] = torch.empty(need + 256, dtype=torch.uint8, device=self.device)
         return ws
 
     def _channels(self, channels):
@@ -504,7 +537,7 @@ class FfnLayer:
         b, e = self._channels(channels)
         m = x.size(0)
         if y is None:
-            y = torch.empty((m, self.hidden), dtype=x.dtype, device=x.device)
+            y = _result((m, self.hidden), x.dtype, x.device, stream)
         if workspace is None:
             workspace = self.workspace(m, stream)
         wp, wb = _aligned(workspace)
@@ -527,8 +560,8 @@ class FfnLayer:
             key = ("block", _stream(stream, self.device))
             workspace = self._ws.get(key)
             if workspace is None or workspace.numel() < need + 256:
-                workspace = torch.empty(need + 256, dtype=torch.uint8, device=self.device)
-                self._ws[key] = workspace
+                with _on(stream, self.device):
+                    workspace = self._ws[key] = torch.empty(need + 256, dtype=torch.uint8, device=self.device)
         wp, wb = _aligned(workspace)
         _call(_lib.load().hm_ffn_block_forward(self._h, _ptr(x), x.stride(0), _ptr(norm_weight), eps, m, wp, wb,
                                                _stream(stream, x.device)))
@@ -538,7 +571,7 @@ class FfnLayer:
         b, e = self._channels(channels)
         m = x.size(0)
         if act is None:
-            act = torch.empty((m, e - b), dtype=x.dtype, device=x.device)
+            act = _result((m, e - b), x.dtype, x.device, stream)
         ws = self.workspace(m, stream)
         wp, wb = _aligned(ws)
         _call(_lib.load().hm_ffn_gate_up(self._h, _ptr(act), act.stride(0), _ptr(x), x.stride(0), m, b, e, wp, wb,
@@ -549,7 +582,7 @@ class FfnLayer:
         b, e = self._channels(channels)
         m = act.size(0)
         if y is None:
-            y = torch.empty((m, self.hidden), dtype=act.dtype, device=act.device)
+            y = _result((m, self.hidden), act.dtype, act.device, stream)
         ws = self.workspace(m, stream)
         wp, wb = _aligned(ws)
         _call(_lib.load().hm_ffn_down(self._h, _ptr(y), y.stride(0), _ptr(act), act.stride(0), m, b, e, wp, wb, _stream(stream, act.device)))
@@ -606,14 +639,15 @@ def ffn_partitioned(layer, x, partition, stream=None):
     if partition.intermediate_channels != layer.inter:
         raise ValueError("partition width must equal the intermediate FFN width")
     partials = {}
-    for dev, (b, e) in partition.slices.items():
-        if b == e:
-            partials[dev] = torch.zeros((x.size(0), layer.hidden), dtype=x.dtype, device=x.device)
-        else:
-            partials[dev] = layer.forward(x, channels=(b, e), stream=stream)
-    reduced = torch.zeros((x.size(0), layer.hidden), dtype=x.dtype, device=x.device)
-    residual_add2(reduced, partials["gpu"], partials["npu"], stream=stream)
-    return reduced, partials
+    with _on(stream, x.device):
+        for dev, (b, e) in partition.slices.items():
+            if b == e:
+                partials[dev] = torch.zeros((x.size(0), layer.hidden), dtype=x.dtype, device=x.device)
+            else:
+                partials[dev] = layer.forward(x, channels=(b, e), stream=stream)
+        reduced = torch.zeros((x.size(0), layer.hidden), dtype=x.dtype, device=x.device)
+        residual_add2(reduced, partials["gpu"], partials["npu"], stream=stream)
+    return _handed_over(reduced, stream), {dev: _handed_over(t, stream) for dev, t in partials.items()}
 
 
 def ffn_row_split(layer, x, y, other_rows, stream=None):

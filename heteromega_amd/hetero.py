@@ -86,7 +86,7 @@ def hetero_linear(out, x, value, w0, w1=None, k=None, stream=None):
     vp = ctypes.byref(value) if value is not None else None
     h1 = w1._h if w1 is not None else None
     need = lib.hm_linear_split_workspace_bytes(vp, w0._h, h1, m, k, n)
-    ws = _workspace(need, x.device)
+    ws = _workspace(need, x.device, stream)
     wp, wb = _aligned(ws)
     _call(lib.hm_linear_split(vp, w0._h, h1, _ptr(out), out.stride(0), _ptr(x), x.stride(0), m, k, n, wp, wb, _stream(stream, x.device)))
     return out

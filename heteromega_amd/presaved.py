@@ -241,6 +241,11 @@ def load_ffn_layer(directory, layer, manifest=None, dtype=torch.bfloat16, device
         raise ValueError(f"pre-saved weights: no layer {layer} in {directory}")
     hidden, inter = int(m["hidden_size"]), int(m["intermediate_size"])
     device = torch.device(device)
+    with _ffn._on(stream, device):  # the logical form's tensors are made where the repack reads them
+        return _build_ffn_layer(directory, layer, m, hidden, inter, dtype, device, stream)
+
+
+def _build_ffn_layer(directory, layer, m, hidden, inter, dtype, device, stream):
     if m.get("use_packed_weights", True):
         splits = m.get("split_k_by_layer", {}) or {}
         aligns = [pad_alignment(m.get("pad_packed_weights", False), m.get("pad_packed_weights_by_layer"), n) for n in MLP_MATRICES]
