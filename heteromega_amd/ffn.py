@@ -37,10 +37,15 @@ def _hm_dtype(dtype):
 # about as long as its call takes on the host, and the wrapper objects and the Stream object of torch.cuda.current_stream
 # were 2.5 of the 8.7 us of a packed_linear call (24 Q/K/V projections of 5.3 us each: 190 -> 142 us).
 
+# The current stream's handle by device index without a Stream object: not part of torch's public interface, so a torch without it
+# takes the public call.
+_current_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(stream, device=None):
     if stream is None:
-        if device is not None and device.type == "cuda" and device.index is not None:
-            return torch._C._cuda_getCurrentRawStream(device.index)
+        if _current_raw_stream is not None and device is not None and device.type == "cuda" and device.index is not None:
+            return _current_raw_stream(device.index)
         return torch.cuda.current_stream(device).cuda_stream
     if isinstance(stream, torch.cuda.Stream):
         return stream.cuda_stream
