@@ -103,6 +103,16 @@ GemmPlan plan_gemm(const GemmCall &c) {
     return e.plan;
 }
 
+// For tests, which choose their shapes by the launch that they get: the plan of m rows, cols columns (fused: gate and up) and
+// kt K tiles on `cus` CUs as {tile, its row blocks, waves over columns, K groups, LDS buffers, K tiles per barrier, K splits,
+// bytes of partials}. Host code only, and not part of the C ABI.
+extern "C" void hm_gemm_plan_of(int64_t m, int64_t cols, int64_t kt, int64_t cus, int32_t large_scales, int64_t out[8]) {
+    const GemmPlan p = plan_uncached(m, cols, kt, cus, large_scales != 0);
+    const GemmTile t = p.cfg < 0 ? GemmTile{} : kGemmTiles[p.cfg];
+    const int64_t v[8] = {p.cfg, t.rbw, t.wn, t.wk, t.depth, t.kpb, p.splits, static_cast<int64_t>(p.partial_bytes)};
+    std::copy(v, v + 8, out);
+}
+
 size_t gemm_partial_bound(int64_t m, int64_t cols, int64_t kt) {
     return kt < 4 ? 0 : std::min(kGemmPartialMax, static_cast<size_t>(std::min(kMaxSplits, kt / 2) * m * cols) * sizeof(float));
 }

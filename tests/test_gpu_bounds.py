@@ -49,12 +49,14 @@ def _weights(oracle, hm, device, k, n, group, dtype, seed):
     return w, hm.RepackedMatrix.from_logical(*logical_to_device(w, dtype, device), group, dtype=TORCH[dtype])
 
 
-# (k, n, m) and the launch each gets from the planner: 64 x 128 tiles with K split in 2, 2, 4 (m = 37, 100, 300 at
-# n = 1024: 8, 16 and 40 workgroups); 64 x 128 tiles, 160 workgroups, no split (m = 600); 128 x 256 tiles, 256
-# workgroups, no split (m = 1999); 128 x 128 tiles, 192 workgroups, no split (m = 300 at n = 8192); the decode
-# GEMV (m = 5, 16). Every GEMM case has a last row tile that ends inside the tile.
+# (k, n, m) and the launch each gets from the planner: one launch with four K groups (m = 37, 100, 300 at n = 1024) or two
+# (m = 600; m = 300 at n = 8192), without K groups (m = 1999), the decode GEMV (m = 5, 16), and K splits of 8, 2 and 4 with fp32
+# partials (the last three, GEMM_SPLITS). Every GEMM case but the last has a last row tile that ends inside the tile.
 CASES = [(2048, 1024, 37), (2048, 1024, 100), (4096, 1024, 300), (2048, 2048, 600), (2048, 4096, 1999), (2048, 8192, 300),
-         (1024, 512, 5), (2048, 1024, 16)]
+         (1024, 512, 5), (2048, 1024, 16), (4096, 512, 100), (6144, 4096, 300), (8192, 1024, 600)]
+# (rows, columns, K, K splits) of the GEMM calls here that write partials.
+GEMM_SPLITS = [(100, 512, 4096, 8), (300, 4096, 6144, 2), (600, 1024, 8192, 4), (37, 512, 4096, 8), (37, 512, 6144, 12), (300, 640, 5120, 5),
+               (300, 640, 10240, 5), (144, 2048, 6144, 5), (40, 1024, 4096, 8), (100, 2048, 8192, 4)]
 
 
 @pytest.mark.parametrize("dtype", ["fp16", "bf16"])
@@ -81,7 +83,17 @@ def test_linear_writes_only_its_block(oracle, hm, device, dtype, k, n, m):
 
 @pytest.mark.parametrize("m", [1, 7, 37, 300])
 def test_k_split_pair_accumulate_writes_only_its_block(oracle, hm, device, m):
-    dtype, k0, k1, n = "fp16", 1536, 2560, 1024
+    _pair_writes_only_its_block(oracle, hm, device, m, 1536, 2560, 1024)
+
+
+@pytest.mark.parametrize("m,k0,k1,n", [(37, 4096, 6144, 512), (300, 10240, 5120, 640)])
+def test_k_split_pair_split_sums_write_only_their_block(oracle, hm, device, m, k0, k1, n):
+    # both shares' GEMMs split K: the second one's split sum adds into the output
+    _pair_writes_only_its_block(oracle, hm, device, m, k0, k1, n)
+
+
+def _pair_writes_only_its_block(oracle, hm, device, m, k0, k1, n):
+    dtype = "fp16"
     w0, r0 = _weights(oracle, hm, device, k0, n, 128, dtype, 1)
     w1, r1 = _weights(oracle, hm, device, k1, n, 128, dtype, 2)
     rng = np.random.default_rng(100 + m)
@@ -105,7 +117,17 @@ def test_k_split_pair_accumulate_writes_only_its_block(oracle, hm, device, m):
 # (1000, 3584): the fused gate_up GEMM runs 8 row tiles of 128, the last one ragged.
 @pytest.mark.parametrize("m,inter", [(1, 2816), (3, 2816), (37, 2816), (333, 2816), (1000, 3584)])
 def test_ffn_writes_only_its_block(oracle, hm, device, m, inter):
-    dtype, hidden, group = "bf16", 2048, 128
+    _ffn_writes_only_its_block(oracle, hm, device, m, 2048, inter)
+
+
+# The gate_up GEMM splits K (SwiGLU in the split sum), or the down GEMM does.
+@pytest.mark.parametrize("m,hidden,inter", [(144, 6144, 1024), (40, 4096, 512), (40, 1024, 4096), (100, 2048, 8192)])
+def test_ffn_split_sums_write_only_their_block(oracle, hm, device, m, hidden, inter):
+    _ffn_writes_only_its_block(oracle, hm, device, m, hidden, inter)
+
+
+def _ffn_writes_only_its_block(oracle, hm, device, m, hidden, inter):
+    dtype, group = "bf16", 128
     rng = np.random.default_rng(7)
     ws_ = [oracle.random_weights(rng, hidden, inter, group, dtype), oracle.random_weights(rng, hidden, inter, group, dtype),
            oracle.random_weights(rng, inter, hidden, group, dtype)]

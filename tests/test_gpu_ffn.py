@@ -9,6 +9,10 @@ from gpu_util import TORCH, assert_close, dev, dev_bits, host_bits, host_f64, lo
 
 pytestmark = pytest.mark.gpu
 
+# (rows, columns, K, K splits) of the GEMM calls that the tests here have split K.
+GEMM_SPLITS = [(512, 4096, 14336, 2), (256, 4096, 14336, 4), (512, 5120, 13824, 3), (144, 2048, 6144, 5), (100, 1024, 4096, 4), (40, 4608, 5120, 7),
+               (40, 1024, 4096, 8)]
+
 _CACHE = {}
 
 
@@ -59,9 +63,9 @@ def test_ffn_prefill_llama3_8b(oracle, hm, device, dtype, m, rows):
     torch.cuda.synchronize()
     sel = np.arange(m) if rows is None else np.sort(rng.choice(m, rows, replace=False))
     assert_close(oracle, host_f64(y)[sel], _ffn_ref(oracle, x64[sel], wf, dtype), dtype, f"Llama-3-8B FFN prefill M={m}")
-    # rows are independent: a row block alone gives the same bits where neither call splits K (M = 2048 and its
+    # rows are independent: a row block alone gives the same bits where neither call divides K (M = 2048 and its
     # 1536-row block), and equal within rounding where one does (M = 512: both down GEMMs split, differently; a
-    # 1024-row block: its down GEMM splits K in two)
+    # 1024-row block: its down GEMM has two K groups)
     if m == 2048:
         y_part = layer.forward(x[256:1792].contiguous())
         torch.cuda.synchronize()
@@ -78,9 +82,9 @@ def test_ffn_prefill_llama3_8b(oracle, hm, device, dtype, m, rows):
 @pytest.mark.parametrize("dtype", ["fp16", "bf16"])
 @pytest.mark.parametrize("m", [40, 100])
 def test_ffn_gemm_k_split(oracle, hm, device, dtype, m):
-    # Small GEMM grids split K: hidden 2688 = 21 K tiles (the fused gate_up's 36 column tiles split 11 + 10,
-    # SwiGLU applied after the split sum), intermediate 2304 = 18 K tiles (the down's 21 column tiles split
-    # 9 + 9); M not a multiple of the 64-row tile. All rows against the oracle, and the bits equal a repeat call.
+    # Small GEMM grids divide K over four K groups in a workgroup: hidden 2688 = 21 K tiles (6 + 5 + 5 + 5, SwiGLU after
+    # their sums met), intermediate 2304 = 18 K tiles (5 + 5 + 4 + 4); M not a multiple of the row tile. All rows against
+    # the oracle, and the bits equal a repeat call.
     layer, _, wf = _layer(oracle, hm, device, 2688, 2304, 128, dtype, 4)
     rng = np.random.default_rng(25 + m)
     x64, x = make_x(oracle, rng, m, 2688, dtype, device)
@@ -88,6 +92,21 @@ def test_ffn_gemm_k_split(oracle, hm, device, dtype, m):
     y2 = layer.forward(x)
     torch.cuda.synchronize()
     assert_close(oracle, host_f64(y), _ffn_ref(oracle, x64, wf, dtype), dtype, f"K-split FFN M={m}")
+    assert torch.equal(y, y2)
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("m,hidden,inter", [(144, 6144, 1024), (100, 4096, 512), (40, 5120, 2304), (40, 1024, 4096)])
+def test_ffn_gemm_split_sum(oracle, hm, device, dtype, m, hidden, inter):
+    # Small grids over a long K write fp32 partials of 5, 4 and 7 K splits for gate_up (SwiGLU applied after the split sum) or
+    # of 8 for the down, each split with K groups (40 K tiles in 7 x 2 runs of 2 and 3). All rows against the oracle.
+    layer, _, wf = _layer(oracle, hm, device, hidden, inter, 128, dtype, 5)
+    rng = np.random.default_rng(26 + m)
+    x64, x = make_x(oracle, rng, m, hidden, dtype, device)
+    y = layer.forward(x)
+    y2 = layer.forward(x)
+    torch.cuda.synchronize()
+    assert_close(oracle, host_f64(y), _ffn_ref(oracle, x64, wf, dtype), dtype, f"split-sum FFN {hidden}x{inter} M={m}")
     assert torch.equal(y, y2)
 
 

@@ -1,6 +1,5 @@
-"""GPU: the MFMA GEMM (more than 16 rows) at the edges of its pipeline and tiles: K runs shorter than the pipeline is deep and with
-every remainder of its unrolled loop, and row and column counts on both sides of every tile height, with K groups of unequal length
-and K splits, against the float64 oracle."""
+"""GPU: the MFMA GEMM (more than 16 rows) at short K runs, at bf16 scales of any size, and at row counts on both sides of 32 to 128
+rows on narrow matrices, against the float64 oracle. Every tile shape at every length of its K runs: test_gpu_gemm_plans.py."""
 
 import numpy as np
 import pytest
@@ -119,9 +118,9 @@ def test_bf16_large_scales_in_a_layer(oracle, hm, device, source):
 @pytest.mark.parametrize("dtype", ["fp16", "bf16"])
 @pytest.mark.parametrize("k,n,group", [(1152, 384, 32), (1408, 128, 64), (2688, 1024, 128), (1024, 6144, 64)])
 def test_tile_edges(oracle, hm, device, k, n, group, dtype):
-    # Rows on both sides of the tile heights (32 to 128 in steps of 16, one tile and several) in a frame that has to stay
-    # untouched; 9, 11 and 21 K tiles do not divide into the K groups and splits, and 128 and 384 columns leave only the
-    # narrow tiles. The second share of a K-split pair adds into its output through the same tiles.
+    # Rows on both sides of 32 to 128 in steps of 16 and beyond, in a frame that has to stay untouched; 9, 11 and 21 K tiles do
+    # not divide into the K groups. These matrices mostly take the 32- and 48-row tiles (the others: test_gpu_gemm_plans.py).
+    # The second share of a K-split pair adds into its output through the same tiles.
     rng = np.random.default_rng(330 + k + n)
     w_np = oracle.random_weights(rng, k, n, group, dtype)
     w = hm.RepackedMatrix.from_logical(*logical_to_device(w_np, dtype, device), group, dtype=TORCH[dtype])
@@ -144,7 +143,7 @@ def test_tile_edges(oracle, hm, device, k, n, group, dtype):
 @pytest.mark.parametrize("dtype", ["fp16", "bf16"])
 @pytest.mark.parametrize("hidden,inter,group", [(1152, 1408, 128), (2048, 8192, 64)])
 def test_tile_edges_fused(oracle, hm, device, hidden, inter, group, dtype):
-    # The fused gate_up (SwiGLU after the K groups' exchange, or in the split sum) at the tile heights.
+    # The fused gate_up, SwiGLU after the K groups' exchange.
     rng = np.random.default_rng(350 + hidden)
     ws = [oracle.random_weights(rng, hidden, inter, group, dtype), oracle.random_weights(rng, hidden, inter, group, dtype),
           oracle.random_weights(rng, inter, hidden, group, dtype)]

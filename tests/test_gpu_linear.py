@@ -10,6 +10,11 @@ from gpu_util import TORCH, assert_close, dev, host_f64, logical_to_device, make
 
 pytestmark = pytest.mark.gpu
 
+# (rows, columns, K, K splits) of the GEMM calls that the tests here have split K, or name as unsplit.
+GEMM_SPLITS = [(17, 1024, 2048, 1), (100, 512, 4096, 8), (130, 768, 2560, 1), (257, 1280, 3072, 1), (300, 4096, 6144, 2), (64, 128, 1024, 1),
+               (1000, 2048, 1024, 1), (33, 384, 2048, 1), (17, 1024, 8192, 8), (33, 384, 6144, 12), (130, 768, 5120, 7), (37, 512, 4096, 8),
+               (37, 512, 6144, 12), (300, 640, 5120, 5), (300, 640, 10240, 5)]
+
 
 def _matrix(oracle, hm, rng, k, n, group, dtype, device):
     w_np = oracle.random_weights(rng, k, n, group, dtype)
@@ -172,7 +177,7 @@ def test_concat_qkv_equals_separate(oracle, hm, device, m):
     # one matrix and one launch. Bit for bit against three launches at one row and where no GEMM launch splits K
     # (M = 4096 here: an output column's sum then does not depend on the other columns); within tolerance at
     # 2..16 rows, where the GEMV's K split follows the matrix width, and at M = 37..2048, where the narrow K/V
-    # launches (small grids) split K and the wide one does not. The concatenated planes decode to the parts'
+    # launches (small grids) divide K otherwise than the wide one. The concatenated planes decode to the parts'
     # logical tensors side by side.
     rng = np.random.default_rng(120)
     k, g, dtype = 4096, 128, "fp16"
@@ -207,8 +212,8 @@ def test_linear_k_split_pair(oracle, hm, device, dtype, m, k0, k1):
     # (out.add_(temp), here torch's add of two separate launches), and within tolerance of the oracle's
     # round(round(a) + round(b)). At one row both shares run in one launch with the longer share's wave split,
     # so their sums take the separate launches' order (and bits) when k0 == k1 and within rounding otherwise.
-    # From 4 rows the second share adds into the output in the split sums (M = 4, 16; the GEMM at M = 37 and
-    # 512 when its 20 K tiles split) or in the GEMM epilogue, bit for bit.
+    # From 4 rows the second share adds into the output in the split sums (M = 4, 16) or in the GEMM epilogue, bit
+    # for bit (in the GEMM's split sums: test_linear_k_split_pair_split_sums).
     rng = np.random.default_rng(140 + m + k0)
     n, g = 1024, 128
     w0_np, w0 = _matrix(oracle, hm, rng, k0, n, g, dtype, device)
@@ -233,21 +238,44 @@ def test_linear_k_split_pair(oracle, hm, device, dtype, m, k0, k1):
             hm.packed_linear_k_split(y, x, w0, w1, k0=k0 - 64)
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("m,k0,k1,n", [(37, 4096, 6144, 512), (300, 5120, 10240, 640)])
+def test_linear_k_split_pair_split_sums(oracle, hm, device, dtype, m, k0, k1, n):
+    # Both shares' GEMMs split K (8 and 12, 5 and 5 splits): the second one's split sum adds its rounded result into the
+    # first one's, bit for bit as two separate launches and torch's add.
+    rng = np.random.default_rng(150 + m)
+    w0_np, w0 = _matrix(oracle, hm, rng, k0, n, 128, dtype, device)
+    w1_np, w1 = _matrix(oracle, hm, rng, k1, n, 128, dtype, device)
+    x64, x = make_x(oracle, rng, m, k0 + k1, dtype, device)
+    y = torch.full((m, n), float("nan"), dtype=TORCH[dtype], device=device)
+    hm.packed_linear_k_split(y, x, w0, w1)
+    y0 = hm.packed_linear(torch.empty((m, n), dtype=TORCH[dtype], device=device), x[:, :k0], w0)
+    y1 = hm.packed_linear(torch.empty((m, n), dtype=TORCH[dtype], device=device), x[:, k0:], w1)
+    torch.cuda.synchronize()
+    assert torch.equal(y, y0 + y1)
+    a = oracle.round_to((x64[:, :k0] @ oracle.weights_f64(*w0_np, 128, dtype)).astype(np.float32), dtype).astype(np.float64)
+    b = oracle.round_to((x64[:, k0:] @ oracle.weights_f64(*w1_np, 128, dtype)).astype(np.float32), dtype).astype(np.float64)
+    assert_close(oracle, host_f64(y), a + b, dtype, f"K split {k0}+{k1} M={m}")
+
+
 @pytest.mark.parametrize("m,k,n,col,g,dtype", [
-    (17, 2048, 1024, 0, 128, "fp16"),     # 8 workgroups: K split in 2 (8 tiles each)
-    (100, 4096, 512, 0, 64, "bf16"),      # group 64, 8 workgroups: K split in 4
-    (130, 2560, 768, 0, 32, "fp16"),      # group 32, 18 workgroups: 20 K tiles split 10 + 10
-    (257, 3072, 1280, 0, 64, "bf16"),     # 50 workgroups: 24 K tiles split in 3
-    (300, 6144, 4096, 0, 128, "fp16"),    # 160 four-wave workgroups: split in 2 toward two per CU
+    (17, 2048, 1024, 0, 128, "fp16"),     # four K groups of 4 K tiles, no split
+    (100, 4096, 512, 0, 64, "bf16"),      # group 64: 8 K splits of two K groups
+    (130, 2560, 768, 0, 32, "fp16"),      # group 32: four K groups of 5 K tiles
+    (257, 3072, 1280, 0, 64, "bf16"),     # four K groups of 6 K tiles
+    (300, 6144, 4096, 0, 128, "fp16"),    # 80-row tiles: 2 K splits of two K groups
     (300, 6144, 4096, 0, 128, "bf16"),
-    (64, 1024, 128, 0, 128, "fp16"),      # 8 K tiles: too few to split
-    (1000, 1024, 2048, 0, 128, "fp16"),   # 256 four-wave workgroups, 8 K tiles: no split
-    (33, 2048, 384, 256, 128, "fp16"),    # a column range on the GEMM path, split in 2
+    (64, 1024, 128, 0, 128, "fp16"),      # four K groups of 2 K tiles, the fewest
+    (1000, 1024, 2048, 0, 128, "fp16"),   # 64-row tiles: two K groups of 4 K tiles
+    (33, 2048, 384, 256, 128, "fp16"),    # a column range on the GEMM path
     (9, 2048, 96, 512, 128, "bf16"),      # a column range on the GEMV path
+    (17, 8192, 1024, 0, 64, "bf16"),      # 8 K splits of four K groups of 2 K tiles
+    (33, 6144, 384, 256, 128, "fp16"),    # a column range with 12 K splits, the most
+    (130, 5120, 768, 0, 32, "bf16"),      # 7 K splits of two K groups: 40 K tiles in 14 runs of 2 and 3
 ])
 def test_linear_planner_shapes(oracle, hm, device, m, k, n, col, g, dtype):
-    # Launch plans across the GEMM's K-split rules (small grids toward 256 workgroups, 4-wave grids toward two
-    # per CU, ragged splits, group 32 / 64, column ranges) against the oracle on every row.
+    # Launch plans across the GEMM's K groups and K splits (ragged ones, group 32 / 64, column ranges) against the oracle
+    # on every row.
     rng = np.random.default_rng(160 + m + k // 128)
     w_np, w = _matrix(oracle, hm, rng, k, col + n + 128, g, dtype, device)
     x64, x = make_x(oracle, rng, m, k, dtype, device)
