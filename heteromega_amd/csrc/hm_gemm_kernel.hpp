@@ -12,12 +12,14 @@
 // dequantized B operand feeds RBW MFMAs (8 at 128 rows: about two VALU instructions per MFMA). The activation tile
 // (16 RBW x 128 per K tile and K group) goes from memory straight into LDS (buffer_load ... lds, no registers) and
 // serves its group's WN waves; its 16-byte chunks are XOR-swizzled by row so that an MFMA operand read touches 16
-// distinct bank groups; one barrier per K tile (per two K tiles for the 256-column tiles).
+// distinct bank groups; one barrier per K tile, per two K tiles for the 256-column tiles, or two per K tile where LDS has room
+// for two whole tiles only, which then lie in four buffers of half a K tile (64 K) each.
 //
 // Software pipeline: while the MFMAs of 32-K step mu run, the VALU builds the B operands of step mu + 1 (of the
 // next K tile at mu = 3) and the LDS delivers the activation fragments of step mu + 1; sched_group_barrier
 // interleaves one MFMA with its share of the VALU instructions. K tile kt + LOOK's weights and activations are
-// requested at the start of K tile kt: LOOK = DEPTH - 1 with one barrier per K tile, 2 (four buffers) with one per two.
+// requested at the start of K tile kt: LOOK = DEPTH - 1 with one barrier per K tile, 2 (four buffers) with one per two. With
+// half tiles the weights are requested two K tiles ahead and the activations three half tiles ahead.
 //
 // Tiles are dealt to XCDs in contiguous runs (workgroup i runs on XCD i % 8 on an MI355X) of an order that walks bands of 4
 // row tiles column by column, so the workgroups resident on one XCD share both activation rows and weight
@@ -160,10 +162,10 @@ __global__ void __launch_bounds__(WN * WK * 64) __attribute__((amdgpu_waves_per_
     constexpr int ADMA = (TRANSFERS + WN - 1) / WN; // per wave (past the last: it is repeated, the same bytes to the same place)
     static_assert(WK == 1 || WK == 2 || WK == 4, "K groups");
     static_assert(WK == 1 || KPB < 2, "K groups whose runs differ by a K tile pass the same barriers");
-    // K tiles in flight: DEPTH - 1 tiles ahead of the one being multiplied, each with its weights in registers
-    // and its activations in one of DEPTH LDS buffers. Per K tile a wave issues NB weight/record loads and ADMA
-    // activation transfers, in that order; all of them count in vmcnt, in order.
-    static_assert(DEPTH >= 2 && DEPTH <= 4, "pipeline depth");
+    // K tiles in flight: LOOK tiles ahead of the one being multiplied, each with its weights in registers and its
+    // activations in one of DEPTH LDS buffers. Per K tile a wave issues NB weight/record loads and ADMA activation
+    // transfers, in that order; all of them count in vmcnt, in order.
+    static_assert(DEPTH == 3 || DEPTH == 4, "pipeline depth");
     // KPB = 2: one barrier per two K tiles. Four LDS buffers, K tiles requested two ahead; the barrier after each odd
     // K tile waits for everything in flight (the next two tiles), and the buffer an iteration fills two tiles ahead was
     // last read before the previous barrier.
@@ -179,11 +181,11 @@ __global__ void __launch_bounds__(WN * WK * 64) __attribute__((amdgpu_waves_per_
     constexpr int AHEAD = KPB == 2 ? 0 : (DEPTH - 2) * (NB + ADMA); // loads issued after tile kt + 1's activations at iteration kt
     // Activation tile of one K tile: BM rows of 128 halves (256 B), 16-byte chunks XOR-swizzled by row
     // (chunk c of row r at slot c ^ (r % 16)), so the 16 rows one MFMA operand read touches fall on distinct banks.
-    // Two separate arrays (not one [2][...]) so that the compiler can tell the buffers apart and does not
+    // Separate arrays (not one [DEPTH][...]) so that the compiler can tell the buffers apart and does not
     // make reads of one wait for the transfers into the other.
     __shared__ __align__(1024) uint8_t as0[BUF];
     __shared__ __align__(1024) uint8_t as1[BUF];
-    __shared__ __align__(1024) uint8_t as2[DEPTH > 2 ? BUF : 16];
+    __shared__ __align__(1024) uint8_t as2[BUF];
     __shared__ __align__(1024) uint8_t as3[DEPTH > 3 ? BUF : 16];
 
     const int tid = threadIdx.x;
@@ -345,11 +347,8 @@ __global__ void __launch_bounds__(WN * WK * 64) __attribute__((amdgpu_waves_per_
             load_a(ktn, (U + LOOK) % DEPTH);
         }
         // The next tile's activations: this wave's transfers done, then everyone's (KPB = 2: after each odd tile, for the
-        // next two). Every read of this tile is done too, so the slot that the next iteration fills is free. With tiles
-        // requested two or more ahead this stands before the last step's MFMAs, which then cover the LDS latency of the
-        // next tile's first fragments (against behind them, the same bits: Llama-3-8B layer at M = 2048 586 -> 578 us, at
-        // 512 180 -> 177); with one tile ahead the transfers need the whole iteration (M = 100, 200: 3% slower there).
-        constexpr bool kEarly = DEPTH > 2;
+        // next two). Every read of this tile is done too, so the slot that the next iteration fills is free. This stands
+        // before the last step's MFMAs, which then cover the LDS latency of the next tile's first fragments.
         auto next_tile = [&]() __attribute__((always_inline)) {
             if constexpr (KPB == 1 || kOdd) {
                 wait_vmcnt<ISSUED>();
@@ -368,10 +367,8 @@ __global__ void __launch_bounds__(WN * WK * 64) __attribute__((amdgpu_waves_per_
                 // iteration ago, before nxt's and this iteration's transfers; at an even kt the barrier before this
                 // iteration already waited for them.
                 wait_vmcnt<KPB == 1 ? ADMA + ISSUED : !kOdd ? ADMA + NB : kRequest ? 2 * ADMA + NB : ADMA>();
-                if constexpr (kEarly) {
-                    next_tile();
-                    read_a((U + 1) % DEPTH, 0, fn);
-                }
+                next_tile();
+                read_a((U + 1) % DEPTH, 0, fn);
                 dequant_step(nxt, dq, 0, on);
             }
             // strip-major: the operand of the last strip, finished at the end of the previous step, is needed last
@@ -389,13 +386,7 @@ __global__ void __launch_bounds__(WN * WK * 64) __attribute__((amdgpu_waves_per_
             }
             __builtin_amdgcn_sched_barrier(0);
             op = on;
-            if (mu < 3 || kEarly) {
-                fa = fn;
-            }
-        }
-        if constexpr (!kEarly) {
-            next_tile();
-            read_a((U + 1) % DEPTH, 0, fa);
+            fa = fn;
         }
     };
 
@@ -504,9 +495,7 @@ __global__ void __launch_bounds__(WN * WK * 64) __attribute__((amdgpu_waves_per_
     for (; kt + DEPTH - 1 < nkt; kt += DEPTH) {
         one(kt, std::integral_constant<int, 0>{}, Steady{});
         one(kt + 1, std::integral_constant<int, 1>{}, Steady{});
-        if constexpr (DEPTH > 2) {
-            one(kt + 2, std::integral_constant<int, 2>{}, Steady{});
-        }
+        one(kt + 2, std::integral_constant<int, 2>{}, Steady{});
         if constexpr (DEPTH > 3) {
             one(kt + 3, std::integral_constant<int, 3>{}, Steady{});
         }
@@ -514,10 +503,8 @@ __global__ void __launch_bounds__(WN * WK * 64) __attribute__((amdgpu_waves_per_
     if (kt < nkt) {
         one(kt, std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
     }
-    if constexpr (DEPTH > 2) {
-        if (kt + 1 < nkt) {
-            one(kt + 1, std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{});
-        }
+    if (kt + 1 < nkt) {
+        one(kt + 1, std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{});
     }
     if constexpr (DEPTH > 3) {
         if (kt + 2 < nkt) {
