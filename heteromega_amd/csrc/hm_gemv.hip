@@ -1203,55 +1203,64 @@ GemvPlan plan_gemv_uncached(const GemvCall &c, int64_t cus, bool allow_few = tru
         // sweeps of every (splits, nu, wps) on the gate_up and down projections of Llama-3-8B, Qwen2.5-14B and
         // Llama-3.2-1B at 2, 4, 8, 12 and 16 rows (one graph of 60 launches per shape, the graphs' replays
         // interleaved, weights streamed from HBM).
-        // Where the whole K does not fit LDS the launch splits in any case, and (groups of 64 and 128) 0.09, 0.03, 0.12 and
-        // 0.13 take those weights' places, fitted to the downs at 9 to 16 rows, fp16 and bf16: more splits, of smaller
-        // staged chunks, two of which fit a CU. The downs run mostly 3 to 6% faster: Llama-3-8B at 16 rows 13.0 -> 12.4 us
-        // (fp16), 13.2 -> 12.5 (bf16), Qwen2.5-14B 14.7 -> 14.2 and 15.0 -> 14.0, Llama-3.2-1B 8.8 -> 8.4 and 8.9 -> 8.6
-        // (groups of 32, half the ring: Llama-3-8B at 6 rows 13.6 -> 15.2, so they keep the first weights).
+        // Where the whole K does not fit LDS the launch splits in any case, and (groups of 64 and 128) a second weighing with
+        // 0.09, 0.03, 0.12 and 0.13 in those weights' places decides, fitted to the downs at 9 to 16 rows, fp16 and bf16: more
+        // splits, of smaller staged chunks, two of which fit a CU. The downs run mostly 3 to 6% faster: Llama-3-8B at 16 rows
+        // 13.0 -> 12.4 us (fp16), 13.2 -> 12.5 (bf16), Qwen2.5-14B 14.7 -> 14.2 and 15.0 -> 14.0, Llama-3.2-1B 8.8 -> 8.4 and
+        // 8.9 -> 8.6 (groups of 32, half the ring: Llama-3-8B at 6 rows 13.6 -> 15.2, so they keep the first weights). It
+        // takes at most 8 splits, whose loads the split sum holds in flight at once, and leaves calls alone that take more by
+        // the first weights: with up to 16, up to 3072 columns ran 3 to 18% slower (8192 x 1024 at 9 rows 7.2 -> 8.5 us).
         const bool whole = stage_bytes(c.kt_count) <= kLdsMax;
         const bool deep = !whole && c.w.group > 32;
         const int64_t rows_pad = (c.m + 3) & ~int64_t{3};
         const int gpt = static_cast<int>(128 / c.w.group);
         const int ring = std::max(1, (p.spw == 1 || gpt > 1 ? 4 : 8) / p.spw / (gpt == 4 ? 2 : 1)); // the kernel's KB
-        double best = -1.0;
-        for (int64_t sp = 1; sp <= std::min<int64_t>(c.kt_count, 16); ++sp) {
-            const int64_t ktp = (c.kt_count + sp - 1) / sp;
-            if ((c.kt_count + ktp - 1) / ktp != sp || (sp > 1 && sp * p.groups > kUnitsPerCu * cus)) {
-                continue; // a split count that a smaller count already gives, or partials past the bound
-            }
-            const size_t stage = stage_bytes(ktp);
-            for (int wps = 1; wps <= 4; wps *= 2) {
-                for (int nu = 1; nu <= 8; nu *= 2) {
-                    const int waves = nu * wps;
-                    const size_t lds = std::max(stage, rows_red(wps, nu));
-                    if ((waves != 4 && waves != 8 && waves != 16) || lds > kLdsMax) {
-                        continue;
-                    }
-                    const int64_t wgs = (p.groups + nu - 1) / nu * sp;
-                    const int64_t per_cu = std::min<int64_t>(static_cast<int64_t>(kLdsMax / lds), 16 / waves);
-                    const int64_t rounds = (wgs + cus * per_cu - 1) / (cus * per_cu);
-                    const int64_t tpw = (ktp + wps - 1) / wps;
-                    const double inflight = static_cast<double>(p.groups * sp * wps * std::min<int64_t>(ring, tpw) * p.spw);
-                    const double imb = static_cast<double>((wgs + cus - 1) / cus * cus) / static_cast<double>(wgs);
-                    const double r = inflight / static_cast<double>(kRowsInFlight);
-                    const double partial = sp > 1 ? 16.0 * static_cast<double>(sp * c.m) / static_cast<double>(c.kt_count * 128) : 0.0;
-                    const double cost = imb * (r < 1.0 ? std::sqrt(1.0 / r) : std::pow(r, deep ? 0.09 : 0.05)) *
-                                        (1.0 + (deep ? 0.03 : 0.05) * static_cast<double>(rows_pad) / (4.0 * nu * p.spw)) *
-                                        (1.0 + (deep ? 0.12 : 0.5) * partial) *
-                                        (1.0 + (deep ? 0.13 : 0.25) * static_cast<double>(rounds - 1));
-                    // Candidates come in order of splits, so equal costs keep fewer splits; within the same
-                    // splits an equal cost takes the larger workgroup.
-                    const bool lower = best < 0.0 || cost < best * (1.0 - 1e-9);
-                    const bool tie_bigger = !lower && cost <= best * (1.0 + 1e-9) && sp == p.splits && waves > p.nu * p.wps;
-                    if (lower || tie_bigger) {
-                        best = cost;
-                        p.kt_per_split = ktp;
-                        p.splits = sp;
-                        p.wps = wps;
-                        p.nu = nu;
+        auto weigh = [&](int64_t max_splits, bool deep) {
+            double best = -1.0;
+            for (int64_t sp = 1; sp <= std::min(c.kt_count, max_splits); ++sp) {
+                const int64_t ktp = (c.kt_count + sp - 1) / sp;
+                if ((c.kt_count + ktp - 1) / ktp != sp || (sp > 1 && sp * p.groups > kUnitsPerCu * cus)) {
+                    continue; // a split count that a smaller count already gives, or partials past the bound
+                }
+                const size_t stage = stage_bytes(ktp);
+                for (int wps = 1; wps <= 4; wps *= 2) {
+                    for (int nu = 1; nu <= 8; nu *= 2) {
+                        const int waves = nu * wps;
+                        const size_t lds = std::max(stage, rows_red(wps, nu));
+                        if ((waves != 4 && waves != 8 && waves != 16) || lds > kLdsMax) {
+                            continue;
+                        }
+                        const int64_t wgs = (p.groups + nu - 1) / nu * sp;
+                        const int64_t per_cu = std::min<int64_t>(static_cast<int64_t>(kLdsMax / lds), 16 / waves);
+                        const int64_t rounds = (wgs + cus * per_cu - 1) / (cus * per_cu);
+                        const int64_t tpw = (ktp + wps - 1) / wps;
+                        const double inflight = static_cast<double>(p.groups * sp * wps * std::min<int64_t>(ring, tpw) * p.spw);
+                        const double imb = static_cast<double>((wgs + cus - 1) / cus * cus) / static_cast<double>(wgs);
+                        const double r = inflight / static_cast<double>(kRowsInFlight);
+                        const double partial = sp > 1 ? 16.0 * static_cast<double>(sp * c.m) / static_cast<double>(c.kt_count * 128) : 0.0;
+                        const double cost = imb * (r < 1.0 ? std::sqrt(1.0 / r) : std::pow(r, deep ? 0.09 : 0.05)) *
+                                            (1.0 + (deep ? 0.03 : 0.05) * static_cast<double>(rows_pad) / (4.0 * nu * p.spw)) *
+                                            (1.0 + (deep ? 0.12 : 0.5) * partial) *
+                                            (1.0 + (deep ? 0.13 : 0.25) * static_cast<double>(rounds - 1));
+                        // Candidates come in order of splits, so equal costs keep fewer splits; within the same
+                        // splits an equal cost takes the larger workgroup.
+                        const bool lower = best < 0.0 || cost < best * (1.0 - 1e-9);
+                        const bool tie_bigger = !lower && cost <= best * (1.0 + 1e-9) && sp == p.splits && waves > p.nu * p.wps;
+                        if (lower || tie_bigger) {
+                            best = cost;
+                            p.kt_per_split = ktp;
+                            p.splits = sp;
+                            p.wps = wps;
+                            p.nu = nu;
+                        }
                     }
                 }
             }
+            return best;
+        };
+        const double best = weigh(16, false);
+        if (deep && p.splits <= 8) {
+            weigh(8, true);
         }
         if (best < 0.0) {
             // No candidate within the partial bound: a long K whose staged chunk needs more splits than the bound allows
@@ -1264,7 +1273,7 @@ GemvPlan plan_gemv_uncached(const GemvCall &c, int64_t cus, bool allow_few = tru
         }
         // Narrow projections whose whole K fits LDS run in one unsplit launch: the sum of the partials is a second launch
         // of 2.5-3 us behind a GEMV of 3-5. Each workgroup takes one strip group over the whole K, with 8 waves of at
-        // least 4 K tiles, else 4. fp16 and fused calls take strip pairs; plain bf16 calls, where lone strips stream
+        // least 4 K tiles (2 in groups of 32 and 64), else 4. fp16 and fused calls take strip pairs; plain bf16 calls, where lone strips stream
         // better, single strips (two per workgroup of four waves past one strip per CU), also where the rule above has
         // pairs and does not split. Past one workgroup per CU the staged rows would go round twice (6144 columns in 384
         // workgroups: 12.4 us against 8.0 in 192 of two strips), so wider calls keep the rule above. Measured at 9 / 16
@@ -1276,18 +1285,28 @@ GemvPlan plan_gemv_uncached(const GemvCall &c, int64_t cus, bool allow_few = tru
         //   2048 x 3072  7.8 / 8.0 -> 4.9 / 5.2      7.8 / 8.2 -> 4.8 / 5.0
         //   1024 x 4096  6.7 / 6.9 -> 4.0 / 4.2      6.7 / 7.1 -> 4.0 / 4.1
         // A pair's wave streams twice the tiles: few pairs of a long K (8192 x 2048, groups of 64 at 5 rows: 8.3 -> 9.3; in
-        // single strips of bf16 8.5 -> 7.6) or in groups of 32 (4096 x 1024 fused: 7.6 -> 8.5) stay split.
+        // single strips of bf16 8.5 -> 7.6) or in groups of 32 (4096 x 1024 fused: 7.6 -> 8.5) stay split. Where the lines
+        // lie, as unsplit time over split time on both sides:
+        //   pairs, K of 4224 to 5120: 16 rows 1024 columns 1.11-1.16, 1536 1.07-1.14, 2048 0.99-1.05, 2560 0.96-1.00, 3072
+        //     0.94-0.99; 12 rows 1536 1.05-1.09, 2048 0.95-1.01; 5 to 8 rows 1024 1.03-1.07, 1536 0.89-1.03, 2048 0.92-0.98
+        //   single strips, K of 6656 / 7168 / 7680 to 8192: 512 columns up to 0.97, 1024 0.98-1.03 / 0.99-1.00 / 1.02-1.04,
+        //     1536 up to 0.92; in groups of 32, K of 6144 / 6656: 256 and 512 columns 0.95-1.02 / 1.05-1.10, 1536 up to 0.97
+        // Finer groups take longer per tile and so eight waves from 16 K tiles (3968 x 6144, groups of 32, at 12 rows: split
+        // 10.3 us, unsplit in four waves 12.1, in eight 8.9); in groups of 128, fp16, eight waves of 16 to 28 K tiles are
+        // 0-3% slower than four.
         // (A plan without few rows is made to see whether the rule above splits.)
         const bool pairs = (c.fused || c.w.dtype == HM_FP16) && strips % 2 == 0;
         const int64_t groups = pairs ? strips / 2 : strips;
-        const bool fits = pairs ? groups <= cus && c.kt_count <= 40 && (c.w.group > 32 || 4 * groups >= 3 * cus)
-                                : groups <= 2 * cus && c.kt_count <= 64;
+        const int64_t many = rows_pad / 4 + 1; // sixteenths of the CUs: more rows are staged in longer, by few workgroups as by many
+        const int64_t longest = 4 * groups > cus ? 64 : c.w.group == 32 ? 48 : 8 * groups > cus ? 56 : 64;
+        const bool fits = pairs ? groups <= cus && c.kt_count <= (16 * groups >= many * cus ? 40 : 32) && (c.w.group > 32 || 4 * groups >= 3 * cus)
+                                : groups <= 2 * cus && c.kt_count <= longest;
         if (allow_few && whole && fits && (p.splits > 1 || (!pairs && c.kt_count >= 8))) {
             p.spw = pairs ? 2 : 1;
             p.groups = groups;
             set_splits(1);
             p.nu = groups <= cus ? 1 : 2;
-            p.wps = p.nu == 1 && c.kt_count >= 32 ? 8 : 4;
+            p.wps = p.nu == 1 && c.kt_count >= (c.w.group < 128 ? 16 : 32) ? 8 : 4;
         }
     }
     p.waves = p.units > 0 ? p.units : p.nu * p.wps;
@@ -1352,6 +1371,22 @@ GemvPlan plan_gemv(const GemvCall &c) {
         // a failed host allocation only leaves the plan uncached
     }
     return p;
+}
+
+// For tests, which choose their shapes by the launch that they get: the plan of a call of m rows, n columns (fused: channels)
+// and kt K tiles on `cus` CUs as {on the one-row math, strips per wave, strip groups, K splits, strip groups per workgroup, waves
+// per strip group, units, bytes of partials}. Host code only, and not part of the C ABI.
+extern "C" void hm_gemv_plan_of(int64_t m, int64_t n, int64_t kt, int32_t group, int32_t dtype, int32_t fused, int64_t cus, int64_t out[8]) {
+    GemvCall c;
+    c.w.group = group;
+    c.w.dtype = dtype;
+    c.m = m;
+    c.n = n;
+    c.kt_count = kt;
+    c.fused = fused != 0;
+    const GemvPlan p = plan_gemv_uncached(c, cus);
+    const int64_t v[8] = {p.few || m == 1, p.spw, p.groups, p.splits, p.nu, p.wps, p.units, static_cast<int64_t>(p.partial_bytes)};
+    std::copy(v, v + 8, out);
 }
 
 size_t gemv_pair_spill_bytes(int64_t channels) {
