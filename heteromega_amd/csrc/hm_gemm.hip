@@ -8,8 +8,8 @@ namespace hm {
 namespace {
 
 // K splits and K groups change the order of an output element's sum. Calls of more than kFreeRows rows whose 128 x 128
-// tiles fill the CUs (long K: 1.25 times the CUs) take neither, so that in them a row block, a column range or a
-// concatenated matrix computed alone gives the bits of the whole call.
+// tiles fill the CUs (long K: 1.25 times the CUs) take neither: a row block, a column range or a concatenated matrix computed
+// alone gives the bits of the whole call where both calls are of this kind.
 constexpr int64_t kFreeRows = 256;
 constexpr int64_t kLongK = 64; // K tiles
 constexpr int64_t kMaxSplits = 12;
@@ -21,11 +21,13 @@ bool may_split(int64_t m, int64_t cols, int64_t kt, int64_t cus) {
 
 // Estimated time of a launch in us: what a CU's workgroups take one after the other (each run of `its` K tiles at a cost
 // per tile that grows with the rows, plus what filling the pipeline and writing the tile cost), beside the time the weights
-// take to stream, plus the launch, the exchange between K groups and the split sum. The constants are fitted to some 50000
-// measured launches on three MI355X: gate_up, down, Q/K/V and K/V shapes of Llama-3.2-1B, Llama-3-8B and Qwen2.5-14B, 17 to
-// 2048 rows, fp16 and bf16, every tile shape and 1 to 12 splits. Over them the shape it picks takes 0.9% longer than the
-// fastest one on average (0.5 to 1.3% by card, 1.16 times at worst), and 0.88 of the time of the three shapes and the rules
-// by grid size that it replaced (0.52 to 0.75 for the gate_ups of up to 64 rows, which had taken 128-row tiles).
+// take to stream, plus the launch, the exchange between K groups and the split sum. The constants are fitted to launches
+// measured on three MI355X. Checked by timing every shape it weighs (26398 launches for 324 calls: gate_up, down
+// and Q/K/V of Llama-3.2-1B, Llama-3-8B and Qwen2.5-14B, 17 to 2048 rows, fp16 and bf16): the one it picks takes 0.7% longer
+// than the fastest on average, up to 3% in 295 of the calls, 1.16 times at worst. Over 1040 random calls (512 to 14336
+// columns and K) it takes 0.76 of the time of the three shapes and the rules by grid size that it replaced (0.72 at 17 to 40
+// rows, 0.85 past 520); 16 calls are over 2% slower, nearly all of K up to 1152, where the fit has no shapes, and at worst
+// 7808 x 6272 at 49 rows, groups of 32, 20.8 -> 23.4 us.
 double launch_us(const GemmTile &t, int64_t wgs, int64_t its, int64_t cus, double weight_mb, double partial_mb) {
     const double rounds = static_cast<double>((wgs + cus - 1) / cus);
     const double rb = t.rbw, n = static_cast<double>(its);
