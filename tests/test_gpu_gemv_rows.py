@@ -14,10 +14,12 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["fp16", "bf16"])
 @pytest.mark.parametrize("k,n,group", [
     (128, 16, 32), (384, 48, 64), (1024, 4096, 128), (3968, 4112, 128), (4096, 4096, 64), (4096, 1040, 32), (2688, 8192, 64),
-    (2688, 8208, 128), (5120, 2064, 64), (5248, 512, 32), (8192, 256, 64), (14336, 1024, 128)])
+    (2688, 8208, 128), (5120, 2064, 64), (5248, 512, 32), (8192, 256, 64), (14336, 1024, 128), (2048, 1024, 64), (2176, 528, 32),
+    (3968, 6144, 32), (4608, 2560, 128), (4608, 1024, 64), (7680, 1024, 64)])
 def test_rows(oracle, hm, device, k, n, group, dtype):
-    # 16 to 8208 columns: 1, odd counts, 256, 257, 512 and 513 strips; 1, 3, 8, 31, 32, 40, 41, 64 and 112 K tiles. The frame
-    # around the output has to stay untouched.
+    # 16 to 8208 columns: 1, odd counts, 256, 257, 512 and 513 strips; 1, 3, 8, 31, 32, 40, 41, 64 and 112 K tiles; in groups of 32
+    # and 64 eight waves of 16, 17 and 31 K tiles; 36 and 60 K tiles with enough strips to run unsplit and with too few. The
+    # frame around the output has to stay untouched.
     rng = np.random.default_rng(360 + k + n)
     w_np = oracle.random_weights(rng, k, n, group, dtype)
     w = hm.RepackedMatrix.from_logical(*logical_to_device(w_np, dtype, device), group, dtype=TORCH[dtype])
