@@ -151,9 +151,9 @@ hipError_t launch_gemm(const GemmCall &c, hipStream_t stream) {
     a.xcds = device_topology().xcds;
     const dim3 grid(static_cast<unsigned>(p.tiles_m * p.tiles_n), static_cast<unsigned>(p.splits));
     const int group = static_cast<int>(c.w.group);
-    const hipError_t e = c.w.dtype == HM_FP16  ? launch_gemm_f16(a, group, c.fused, p.cfg, grid, stream)
-                         : c.w.large_scales ? launch_gemm_bf16_large_scales(a, group, c.fused, grid, stream)
-                                            : launch_gemm_bf16(a, group, c.fused, p.cfg, grid, stream);
+    const hipError_t e = c.w.dtype == HM_FP16 ? launch_gemm_f16(a, group, c.fused, p.cfg, grid, stream)
+                         : c.w.large_scales   ? launch_gemm_bf16_large_scales(a, group, c.fused, grid, stream)
+                                              : launch_gemm_bf16(a, group, c.fused, p.cfg, grid, stream);
     if (e != hipSuccess || p.splits == 1) {
         return e;
     }
