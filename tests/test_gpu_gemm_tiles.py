@@ -115,6 +115,42 @@ def test_bf16_large_scales_in_a_layer(oracle, hm, device, source):
     assert_close(oracle, host_f64(y), host_f64(act) @ wd, "bf16", "down of the same layer")
 
 
+@pytest.mark.parametrize("group", [32, 128])
+@pytest.mark.parametrize("m,k,col,n", [(17, 4096, 0, 640), (40, 1280, 128, 256), (130, 4096, 256, 384), (300, 2176, 0, 640)])
+def test_bf16_large_scales_forms(hm, device, m, k, col, n, group):
+    # The large scales' kernel on blocks of a matrix, column ranges, strided rows, K splits and as either share of a K-split pair.
+    # Integer activations times 2^-40 and scales of 2^115 .. 2^120: every sum is exact in fp32, so the output is the exact
+    # result's rounding.
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(328 + m)
+    rows, cols = 4096, 640
+    mats, dense = [], []
+    for lo, hi in ((115, 121), (-8, -4)):
+        q = torch.randint(0, 16, (rows, cols), dtype=torch.uint8, device=device, generator=gen)
+        z = torch.randint(0, 17, (rows // group, cols), dtype=torch.uint8, device=device, generator=gen)
+        s = torch.exp2(torch.randint(lo, hi, (rows // group, cols), device=device, generator=gen).double()).to(torch.bfloat16)
+        mats.append(hm.RepackedMatrix.from_logical(q, s, z, group, dtype=torch.bfloat16))
+        dense.append(((q.view(-1, group, cols).double() - z.view(-1, 1, cols).double()) * s.view(-1, 1, cols).double()).view(rows, cols))
+    wide = torch.randint(-2, 3, (m, k + 64), device=device, generator=gen).to(torch.bfloat16) * 2.0 ** -40
+    x = wide[:, :k]
+    ref = (x.double() @ dense[0][:k, col:col + n]).to(torch.bfloat16)
+    frame = torch.full((m + 1, n + 16), 7.0, dtype=torch.bfloat16, device=device)
+    y = frame[:m, :n]
+    hm.packed_linear(y, x, mats[0], k=k, n=n, col_begin=col)
+    torch.cuda.synchronize()
+    assert torch.equal(y, ref)
+    y.fill_(7.0)
+    assert bool((frame == 7.0).all())
+    both = torch.cat([x, x], dim=1)
+    small = (x.double() @ dense[1][:k, :n]).to(torch.bfloat16)
+    large = (x.double() @ dense[0][:k, :n]).to(torch.bfloat16)
+    for pair in (mats, mats[::-1]):
+        out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=device)
+        hm.packed_linear_k_split(out, both, *pair, k0=k, k1=k, n=n)
+        torch.cuda.synchronize()
+        assert torch.equal(out, large + small)
+
+
 @pytest.mark.parametrize("dtype", ["fp16", "bf16"])
 @pytest.mark.parametrize("k,n,group", [(1152, 384, 32), (1408, 128, 64), (2688, 1024, 128), (1024, 6144, 64)])
 def test_tile_edges(oracle, hm, device, k, n, group, dtype):
